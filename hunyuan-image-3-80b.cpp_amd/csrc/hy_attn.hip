@@ -12,8 +12,9 @@
 //    K in stages of 32 (16) floats DMA-copied into a swizzled LDS ring.  Mid-size
 //    grids (64..1023 tiles): the same kernel as 512 stream-K work groups that split
 //    the tiles' K stages evenly, and gemm_fixup_kernel summing the cut tiles' pieces
-//    in K order.  Small grids: one wave per work group, K in steps of 16 straight
-//    from global memory into registers.
+//    in K order.  17 to 128 rows of A with K % 32 == 0: hy_gemm.hip.  Other small
+//    grids: one wave per work group, K in steps of 16 straight from global memory into
+//    registers.
 //  * rope_qknorm_kernel: one wave per (token, head): rotary embedding (1D positions,
 //    2D tables or none), per-head RMSNorm, written to q [T][nh][hd] and, for key
 //    heads, k / v into a [nkv][L][hd] cache at row pos0 + t.
@@ -464,6 +465,7 @@ hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, fl
         }
         return hipGetLastError();
     }
+    if (gemm_small_ok(M, N, K)) return launch_gemm_small(A, W, R, C, M, N, K, s, ws);
     if (ws && gemm_nt_f32_uses_ws(M, N, K)) {
         p.G = GEMM_SK_GROUPS;
         hipLaunchKernelGGL((gemm_nt_f32_lds_kernel<32, 2, 2>), dim3(p.G), dim3(256), 0, s, p);

@@ -191,6 +191,11 @@ size_t gemm_nt_f32_ws_bytes();
 bool gemm_nt_f32_uses_ws(int M, int N, int K);
 hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                               hipStream_t s, float* ws = nullptr);
+// the same product for 17..128 rows of A (hy_gemm.hip), K a multiple of 32; without ws one
+// tile of 128 W rows per work group
+bool gemm_small_ok(int M, int N, int K);
+hipError_t launch_gemm_small(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
+                             hipStream_t s, float* ws);
 hipError_t launch_rope_qknorm(const RopeNormArgs& a, hipStream_t s);
 // ws: flash_attn_ws_floats(hd, ws_slots) of device scratch, or nullptr (no split over
 // the keys)

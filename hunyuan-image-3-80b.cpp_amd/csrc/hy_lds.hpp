@@ -94,6 +94,11 @@ template <int OFF>
 __device__ __forceinline__ void lds_st128_at(uint32_t base, v4i_t v) {
     asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(base), "v"(v), "i"(OFF) : "memory");
 }
+// ds_write_b64 of two dwords at base + a compile-time byte offset
+template <int OFF>
+__device__ __forceinline__ void lds_st64_at(uint32_t base, uint32_t lo, uint32_t hi) {
+    asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(base), "v"((uint64_t)lo | ((uint64_t)hi << 32)), "i"(OFF) : "memory");
+}
 __device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // wait until at most N of this wave's LDS reads are outstanding (they complete in
 // order); pin each consumed result afterwards (lds_pin)
@@ -106,6 +111,7 @@ __device__ __forceinline__ void lds_wait_upto() {
 // the wait (volatile asm statements keep their program order).
 __device__ __forceinline__ void lds_pin(v4i_t& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void lds_pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void lds_pin(int& v) { asm volatile("" : "+v"(v)); }
 // Force a value to be computed here (before any later volatile asm, e.g. the next
 // round of ds_reads), which bounds how many loaded operands are live at once.
 __device__ __forceinline__ void pin_f32(float& v) { asm volatile("" : "+v"(v)); }

@@ -146,8 +146,8 @@ int hy_model_forward_hidden(hy_model_ctx* ctx, const float* inputs_embeds_dev, u
                             const int32_t* positions_dev, uint32_t n_layers, float* hidden_dev, void* stream);
 
 /* lm_head_f32 (src/hunyuan_full_model.cpp:298-318) and the projections' GEMM:
- * out[t][v] = sum_h x[t][h] * w[v][h] (+ resid[t][v] when resid_dev is not NULL),
- * fp32 MFMA; x [T][hidden], w [vocab][hidden], all device memory; hidden a multiple
+ * out[t][v] = sum_h x[t][h] * w[v][h] (+ resid[t][v] when resid_dev is not NULL), in
+ * fp32 (fp32 MFMA, or exact three-way bf16 splits of the operands); x [T][hidden], w [vocab][hidden], all device memory; hidden a multiple
  * of 16.  Mid-size shapes split the reduction over a per-device scratch that the
  * library allocates on first use and orders between calls with an event: those shapes
  * return HY_ERR_UNSUPPORTED under stream capture (hy_model_forward, whose context

@@ -1,0 +1,64 @@
+"""The fp32 product through bf16 pieces (csrc/hy_gemm.hip), against float64.
+
+Bound: every element adds at most 6 K / 16 matrix-core results (and the K / 32 stage
+pieces of a cut tile) in fp32, each rounding at most 2^-24 of a partial sum that is at
+most S = sum_k |a_k w_k|, and drops piece products below 2^-24 |a_k w_k|:
+|c - exact| <= (6 K / 16 + K / 32 + 4) 2^-24 S.  A first-order term as large again covers
+roundings inside a matrix instruction."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def check(got, x, w, r=None):
+    K = x.shape[1]
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    want = x64 @ w64.T + (0.0 if r is None else r)
+    bound = 2 * (6 * K / 16 + K / 32 + 4) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
+    if r is not None:
+        bound += 2.0 ** -24 * (np.abs(want) + np.abs(r))
+    assert np.all(np.abs(got - want) <= bound)
+
+
+# one to four 32-row tiles and their edges; N below, at and past a 128-row tile; one stage
+# of K, fewer stages than work groups, and ranges that cut every tile
+@pytest.mark.parametrize("M,N,K", [(17, 100, 32), (32, 128, 64), (33, 129, 96), (64, 517, 1024), (65, 257, 4096),
+                                   (96, 6150, 4096), (97, 4096, 512), (128, 10003, 2048)])
+def test_small_batches(gpu, M, N, K):
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, K)).astype(np.float32) * np.exp2(rng.integers(-20, 20, (M, 1))).astype(np.float32)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    check(gpu.lm_head_f32(x, w), x, w)
+    check(gpu.lm_head_f32(x, w, r), x, w, r)
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 300, 256), (128, 9000, 1024)])
+def test_values_without_a_split(gpu, M, N, K):
+    """Infinities, NaNs and values that round up to infinity in bf16 give what an fp32
+    product gives; the other elements keep their bound."""
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    x[3, 7] = np.inf
+    x[5, K - 1] = np.nan
+    w[11, 0] = -np.inf
+    w[N - 1, 9] = np.float32(3.4e38)  # finite; its nearest bf16 is infinity
+    x[:, 9] = np.float32(2.0 ** -40)
+    got = gpu.lm_head_f32(x, w)
+    with np.errstate(all="ignore"):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(got[inf], want[inf].astype(np.float32))
+    rows, cols = [i for i in range(M) if i not in (3, 5)], [j for j in range(N) if j != 11]
+    check(got[np.ix_(rows, cols)], x[rows], w[cols])
+
+
+def test_tiny_values(gpu):
+    """Operands down at 2^-100 keep their significand (bf16 pieces down to denormals)."""
+    rng = np.random.default_rng(2)
+    x = (rng.standard_normal((48, 512)) * 2.0 ** -100).astype(np.float32)
+    w = (rng.standard_normal((200, 512)) * 2.0 ** 20).astype(np.float32)
+    check(gpu.lm_head_f32(x, w), x, w)
