@@ -301,7 +301,10 @@ int forward_impl(hy_moe_ctx* c, uint32_t layer, const float* x, uint32_t T, floa
     const bool mfma = c->path != HY_PATH_VALU && hy::mfma_path_ok(wt, H, I) && mfma_fits &&
                       (c->path == HY_PATH_MFMA || !gemv_batch(wt, T, K, E));
     const int shape = mfma ? hy::mfma_shape(iT, K, E, H, I) : -1;
-    const int NT = mfma ? hy::mfma_shape_tokens(shape) : hy::gemv_tile_tokens();
+    const bool mfma32 = c->path == HY_PATH_AUTO && wt == HY_TYPE_F32 && hy::mfma_f32_ok(iT, K, E, H, I);
+    const int NT = mfma     ? hy::mfma_shape_tokens(shape)
+                   : mfma32 ? hy::mfma_f32_tokens(iT, K, E)
+                            : hy::gemv_tile_tokens();
     // group-limited greedy, dropping and the aux loss take the general routing path
     const bool ext = c->n_group > 0 || c->cfg.drop_tokens || c->cfg.compute_aux_loss;
     // one token: the router logits and the Q8_0 of x in one launch; the gate/up GEMV's
@@ -364,6 +367,19 @@ int forward_impl(hy_moe_ctx* c, uint32_t layer, const float* x, uint32_t T, floa
         HY_TRY(timed(c, hy::KID_DOWN, s, [&] {
             return hy::launch_ffn_down_mfma(wt, shape, routed_bound + shared_tiles, dn_view(c, L), R, c->hq, c->hd, iT, H,
                                             I, E, K, c->y, c->mm_ctr, s);
+        }));
+        HY_TRY(timed(c, hy::KID_COMBINE, s, [&] {
+            return hy::launch_combine(R, c->y, iT, H, K, has_shared, resid, out, s);
+        }));
+        return HY_OK;
+    }
+    if (mfma32) {
+        const int tiles = routed_bound + shared_tiles;
+        HY_TRY(timed(c, hy::KID_UP, s, [&] {
+            return hy::launch_ffn_up_mfma_f32(tiles, gu_view(c, L), R, x, iT, H, I, E, K, c->hf, s);
+        }));
+        HY_TRY(timed(c, hy::KID_DOWN, s, [&] {
+            return hy::launch_ffn_down_mfma_f32(tiles, dn_view(c, L), R, c->hf, iT, H, I, E, K, c->y, s);
         }));
         HY_TRY(timed(c, hy::KID_COMBINE, s, [&] {
             return hy::launch_combine(R, c->y, iT, H, K, has_shared, resid, out, s);

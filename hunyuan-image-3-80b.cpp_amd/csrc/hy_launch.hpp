@@ -113,6 +113,15 @@ hipError_t launch_ffn_down_mfma(int wtype, int shape, int n_tiles_bound, const M
                                 const int8_t* hq, const float* hd, int T, int H, int I, int E, int K, float* y,
                                 int* mm_ctr, hipStream_t s);
 
+// expert products of F32 weights on the fp32 matrix cores (hy_mfma_f32.hip): the decode
+// GEMV's results bit for bit; tiles of mfma_f32_tokens() pairs
+int mfma_f32_tokens(int T, int K, int E);
+bool mfma_f32_ok(int T, int K, int E, int H, int I);
+hipError_t launch_ffn_up_mfma_f32(int n_tiles_bound, const MatView& W, const Routing& R, const float* x, int T, int H,
+                                  int I, int E, int K, float* hf, hipStream_t s);
+hipError_t launch_ffn_down_mfma_f32(int n_tiles_bound, const MatView& W, const Routing& R, const float* hf, int T,
+                                    int H, int I, int E, int K, float* y, hipStream_t s);
+
 // residency (hy_data.hip)
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 hipError_t launch_synth_matrix(int wtype, uint64_t key, float scale, int rows, int cols, int gu_I, uint8_t* qs,
