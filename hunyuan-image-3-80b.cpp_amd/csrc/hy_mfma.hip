@@ -129,22 +129,31 @@ __device__ __forceinline__ int operand_lane_off(int lr, int lg) { return lr * 32
 // Q4_0 unpack of one 64-row chunk by one wave, as contiguous 16-byte stores: lane l
 // writes pieces l and 64 + l of the chunk's int8 operand rows (32 bytes each, halves
 // swizzled by swz_half).  Piece d is half h = (d % 2) ^ (bit 3 of row d / 2) of row
-// d / 2: the values n - 8 of the low (h = 0, elements 0-15) or high (h = 1, elements
+// d / 2: the values of the low (h = 0, elements 0-15) or high (h = 1, elements
 // 16-31) nibbles of the row's 16 stored bytes; lanes 2j and 2j + 1 read the same
 // nibble row.  nib = the chunk's nibble rows + 16 * (l / 2), dst = its int8 rows + 16 l,
-// sh = 4 h (the same for rows l / 2 and 32 + l / 2).
+// sh = 4 - 4 h (the same for rows l / 2 and 32 + l / 2).
+//
+// A weight n - 8 is left in the high nibble of its byte, as the int8 value 16 (n - 8)
+// (n with its top bit flipped is n - 8 in two's complement): a shift and one
+// three-input logic operation per four weights.  Block dots and accumulators come out 16
+// times too large, exactly -- a block dot is at most 16 x 8 x 127 x 32 < 2^24, and the
+// accumulator chain scales by a power of two (its values are multiples of 2^-48, far
+// from denormals) -- and the epilogue multiplies by 1/16.  Against n - 8 itself (five
+// operations per four weights): Q4_0 layers of T = 48 465 -> 454 us, 4096 skewed tokens
+// 3.94 -> 3.92 ms, a decoder layer of T = 300 906 -> 895 us (same box).
+__device__ __forceinline__ int unpack_q4x16(int v, uint32_t sh) {
+    return (int)((((uint32_t)v << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
+}
 __device__ __forceinline__ void unpack_q4_chunk_at(uint32_t nib, uint32_t dst, uint32_t sh) {
     v4i_t w0 = lds_b128_at<0>(nib);
     v4i_t w1 = lds_b128_at<512>(nib);
     lds_wait(w0, w1);
-    auto cv = [sh](int v) {
-        const uint32_t x = ((uint32_t)v >> sh) & 0x0F0F0F0Fu;
-        return (int)(((x | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
-    };
+    auto cv = [sh](int v) { return unpack_q4x16(v, sh); };
     lds_st128_at<0>(dst, v4i_t{cv(w0[0]), cv(w0[1]), cv(w0[2]), cv(w0[3])});
     lds_st128_at<1024>(dst, v4i_t{cv(w1[0]), cv(w1[1]), cv(w1[2]), cv(w1[3])});
 }
-__device__ __forceinline__ uint32_t unpack_q4_shift(int lane) { return 4u * (uint32_t)((lane & 1) ^ ((lane >> 4) & 1)); }
+__device__ __forceinline__ uint32_t unpack_q4_shift(int lane) { return 4u - 4u * (uint32_t)((lane & 1) ^ ((lane >> 4) & 1)); }
 
 // The exact int32 dots of one 32-wide GGUF block over a 32x32 tile (K = 32 is one
 // block): v_mfma_i32_32x32x32_i8 with a zero accumulator.
@@ -492,7 +501,7 @@ __global__ __launch_bounds__(SH::THREADS, SH::WG_PER_CU) void moe_mfma_kernel(Mm
         wait_copies<LOADS, MM_RING - 2>(nstage - 1 - s);
         uint32_t abase;
         if constexpr (Q4) {
-            // nibbles -> int8 (n - 8): wave w converts chunk w, the chunk it copied itself
+            // nibbles -> int8 16 (n - 8): wave w converts chunk w, the chunk it copied itself
             // (row = lane), so its own copies having landed is enough; the result goes to
             // aun[s & 1], last read by stage s - 2's math, which every wave finished before
             // the previous barrier
@@ -520,8 +529,15 @@ __global__ __launch_bounds__(SH::THREADS, SH::WG_PER_CU) void moe_mfma_kernel(Mm
 
     // ---- epilogues: one per 32-token column group of the wave (ag = the rows of the
     // slab's first half, au = the second half)
-    auto epilogue = [&](const float (&ag)[16], const float (&au)[16], int j) {
+    auto epilogue = [&](float (&ag)[16], float (&au)[16], int j) {
         if (j >= n) return;
+        if constexpr (Q4) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                ag[v] *= 0.0625f;
+                au[v] *= 0.0625f;
+            }
+        }
         if (MODE == 0) {
             // ag = gate rows, au = matching up rows of slab (MM_SLABS * rb + sl)
             const int slab = MM_SLABS * rb + sl;
@@ -611,7 +627,7 @@ __global__ __launch_bounds__(256) void gather_act_kernel(const int8_t* __restric
 // raw 16-byte nibble rows, then the GEMM's stage unpack (unpack_q4_chunk_at) -- and the
 // activation block into all 32 token rows of a B tile with the same swizzle, reads its
 // A0 / A1 / B operands at the GEMM's lane offsets (operand_lane_off) and issues the
-// GEMM's two block-dot MFMAs (block_dot_tile).  Every entry of the two 32x32 results
+// GEMM's two block-dot MFMAs (block_dot_tile; Q4_0 dots leave it 16 times too large).  Every entry of the two 32x32 results
 // is the dot of its weight row with the replicated activation block; the one written
 // for (row r, block b) sits in column (r + b) % 32, so that over the rows and blocks
 // every lane and every result register of both tiles is read out.  Rows past `rows`
@@ -662,7 +678,7 @@ __global__ __launch_bounds__(WAVE) void block_dots_mfma_kernel(const uint8_t* __
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             const int rr = g * 64 + 32 * t + i;
-            if (rr < rows && lr == (rr + b) % 32) out[(size_t)rr * nb + b] = t ? S1[v] : S0[v];
+            if (rr < rows && lr == (rr + b) % 32) out[(size_t)rr * nb + b] = (t ? S1[v] : S0[v]) >> (Q4 ? 4 : 0);
         }
     }
 }
