@@ -10,6 +10,15 @@
 // lo lo, is below 2^-24 of the product: no more than one fp32 rounding of it.  Six
 // bf16 MFMAs of 16 k-steps take 6 x 32 cycles where eight fp32 MFMAs of 2 take 8 x 64.
 //
+// These instructions cut the low bits of what they add towards minus infinity (measured: a
+// mean error of -0.21 of the rms error, whatever the result's sign; the fp32 MFMAs show
+// none), and a later average over rows, as in attention, keeps such a mean while it thins
+// out the rest.  So the accumulators hold the sum and its negative in turns (flip_at),
+// with the pieces of A negated alike, and the mean cancels.
+//
+// The split is exact down to 2^-110; below that the last pieces run out of exponent, an
+// absolute error of at most 2^-134 of the operand.
+//
 // Infinities and NaNs have no such split (inf - inf), and a value that rounds up to
 // infinity in bf16 neither: a wave whose accumulators hold a non-finite value after its
 // k-range computes that range again on the fp32 matrix cores (segment_f32), so such
@@ -59,6 +68,13 @@ __device__ __forceinline__ v16f_t mfma_bf16(v4i_t a, v4i_t b, v16f_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0,
                                                    0, 0);
 }
+// Sign turns: PERIOD stages of one sign, the first one half as long, so that the growing
+// means of neighbouring turns cancel.  flip_at: stage d of a range opens a turn;
+// turn_sign: its sign.
+template <int PERIOD>
+__device__ __forceinline__ bool flip_at(int d) { return d % PERIOD == PERIOD / 2; }
+template <int PERIOD>
+__device__ __forceinline__ float turn_sign(int d) { return (d + PERIOD / 2) / PERIOD % 2 ? -1.0f : 1.0f; }
 // finite iff x - x == 0
 __device__ __forceinline__ bool non_finite(float x) { return !(x - x == 0.0f); }
 
@@ -82,6 +98,8 @@ __device__ __forceinline__ bool non_finite(float x) { return !(x - x == 0.0f); }
 constexpr int SK_BN = 128;  // W rows per work group
 constexpr int SK_KC = 32;   // floats of K per stage
 constexpr int SK_D = 2;     // stages of W in flight
+constexpr int SK_TURN = 4;  // stages of one accumulator sign
+static_assert(SK_TURN / 2 % SK_D == 0, "signs turn between unrolled rounds");
 
 struct GemmSmallArgs {
     const float* A;
@@ -161,14 +179,19 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
         load_a(s0);
 #pragma unroll
         for (int d = 0; d < SK_D - 1; d++) load_w(s0 + d, wb[d]);
+        auto negate = [&] {
+#pragma unroll
+            for (int i = 0; i < MT; i++) acc[i] = -acc[i];
+        };
         auto stage = [&](auto dc, int s) {
             constexpr int D = decltype(dc)::value;
             constexpr int BUF = (D & 1) * L::BYTES;  // SK_D is even: D & 1 == (s - s0) & 1
+            const float sgn = turn_sign<SK_TURN>(s - s0);
             // A(s) -> LDS; its buffer was last read in stage s - 2, which every wave had
             // finished before the barrier of stage s - 1
             static_for<MT>([&](auto ic) {
                 constexpr int I = decltype(ic)::value;
-                const Split2 x = split2(ab[I][0], ab[I][1]), y = split2(ab[I][2], ab[I][3]);
+                const Split2 x = split2(sgn * ab[I][0], sgn * ab[I][1]), y = split2(sgn * ab[I][2], sgn * ab[I][3]);
                 static_for<3>([&](auto qc) {
                     constexpr int Q = decltype(qc)::value;
                     lds_st64_at<BUF + Q * L::PIECE + I * 512>(a_dst, x.p[Q], y.p[Q]);
@@ -210,10 +233,13 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
                 __builtin_amdgcn_sched_barrier(0);  // one sub-step's operands live at a time
             });
         };
-        for (int sb = s0; sb < s1; sb += SK_D)
+        for (int sb = s0; sb < s1; sb += SK_D) {
+            if (flip_at<SK_TURN>(sb - s0)) negate();
             static_for<SK_D>([&](auto dc) {
                 if (sb + decltype(dc)::value < s1) stage(dc, sb + decltype(dc)::value);
             });
+        }
+        if (turn_sign<SK_TURN>(s1 - 1 - s0) < 0.0f) negate();
         bool bad = false;
 #pragma unroll
         for (int i = 0; i < MT; i++)
@@ -315,5 +341,337 @@ hipError_t launch_gemm_small(const float* A, const float* W, const float* R, flo
     default: return gemm_small_launch<4>(p, tiles, s);
     }
 }
+
+// ---------------------------------------------------------------- larger batches (M > 128)
+// Work groups of eight waves take tiles of bm <= 64 MT rows of A times 256 rows of W:
+// wave (wm, wn) owns the 32-row subtiles 2 i + wm of A (i < MT) times 64 rows of W.  K
+// advances in stages of 16 floats: every thread loads its float4s of a stage one stage
+// ahead, splits each element once and stores the pieces into a double-buffered LDS stage,
+// so a tile's elements are fetched and split once per work group.  A stage runs in MT
+// groups of 12 MFMAs (one subtile of A, two of W); the next group's operands are read, a
+// share of the next stage is split and stored, under the current group's MFMAs.  The one
+// barrier of a stage stands before its last group, under which the next stage's first
+// operands are read.
+//
+// The tiles x stages units are cut into G equal contiguous ranges as above; an XCD's work
+// groups take neighbouring ranges, and tiles run through eight row tiles of A before the
+// next tile of W, so an XCD's L2 holds what its work groups share.  M is spread evenly over
+// its row tiles (bm a multiple of 32), so no tile is mostly padding.
+constexpr int GS_BN = 256;  // W rows per work group
+constexpr int GS_KC = 16;   // floats of K per stage
+constexpr int GS_THREADS = 512;
+constexpr int GS_TURN = 8;  // stages of one accumulator sign (a multiple of 4)
+
+struct GemmSplitArgs {
+    const float* A;
+    const float* W;
+    const float* R;  // optional: C = R + A.W^T
+    float* C;
+    int M, N, K;
+    int bm;          // rows of A per tile (a multiple of 32)
+    int mt, nt;      // tiles along M and N
+    int G;           // work groups; G = tiles: one whole tile each
+    int qd, rem;     // tiles x stages = G qd + rem: the first rem ranges take qd + 1 units
+    float* part;     // 2 G slots of MT x 64 x 256 floats (unused when G = tiles)
+};
+__device__ __forceinline__ int gs_lo(const GemmSplitArgs& p, int g) { return g * p.qd + min(g, p.rem); }
+__device__ __forceinline__ int gs_owner(const GemmSplitArgs& p, int u) {
+    const int big = p.rem * (p.qd + 1);
+    return u < big ? u / (p.qd + 1) : p.rem + (u - big) / p.qd;
+}
+// row and column tile of tile t
+__device__ __forceinline__ void gs_tile(const GemmSplitArgs& p, int t, int& m, int& n) {
+    const int sg = t / (8 * p.nt), r = t - sg * 8 * p.nt, mw = min(8, p.mt - 8 * sg);
+    m = 8 * sg + r % mw;
+    n = r / mw;
+}
+
+// LDS of one stage: for A and W three pieces of two k-chunks of 8 (chunk h: floats
+// 4 h .. + 3 and 8 + 4 h .. + 3 of a row, the k-slots of MFMA lane half h), each one
+// 16-byte slot per row; the 64 bytes between chunks put the two chunks a wave stores at
+// once on different banks.
+template <int MT>
+struct GsLds {
+    static constexpr int CHUNK_A = MT * 64 * 16 + 64, PIECE_A = 2 * CHUNK_A;
+    static constexpr int CHUNK_W = GS_BN * 16 + 64, PIECE_W = 2 * CHUNK_W;
+    static constexpr int OFF_W = 3 * PIECE_A;
+    static constexpr int BYTES = OFF_W + 3 * PIECE_W;
+    static constexpr int NA = (MT + 1) / 2;  // float4s of A per thread and stage (the last may be half)
+    static constexpr int NC = NA + 2;        // and of A and W
+};
+
+template <int MT>
+__global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmSplitArgs p) {
+    using L = GsLds<MT>;
+    __shared__ __attribute__((aligned(1024))) uint8_t buf[2][L::BYTES];
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int wm = wv / 4, wn = wv % 4;  // waves w and w + 4 share a SIMD: one of each wm
+    const int lr = lane % 32, h = lane / 32;
+    const int M = p.M, N = p.N, K = p.K;
+    const int nst = K / GS_KC;
+    const int mv = (p.bm / 32 - wm + 1) / 2;  // this wave's subtiles of A: MT or MT - 1
+
+    // float4 i of a stage: floats 4 (tid % 4) .. + 3 of tile row 128 i + tid / 4 (A) or
+    // 128 (i - NA) + tid / 4 (W)
+    const int k4 = tid % 4, cr = tid / 4;
+    const int dst = (k4 % 2 ? 1 : 0), sub = 8 * (k4 / 2);
+    uint8_t* const wr_a = buf[0] + dst * L::CHUNK_A + cr * 16 + sub;
+    uint8_t* const wr_w = buf[0] + L::OFF_W + dst * L::CHUNK_W + cr * 16 + sub;
+    const uint8_t* const rd_a = buf[0] + h * L::CHUNK_A + (32 * wm + lr) * 16;
+    const uint8_t* const rd_w = buf[0] + L::OFF_W + h * L::CHUNK_W + (64 * wn + lr) * 16;
+    const bool a_last = 128 * (L::NA - 1) + 16 * wv < p.bm;  // this wave copies the last float4 of A
+
+    // stages [s0, s1) of the tile at (m0, n0) on the fp32 matrix cores (non-finite operands)
+    auto segment_f32 = [&](int m0, int n0, int s0, int s1, v16f_t (&acc)[MT][2]) {
+        const float* w[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) w[j] = p.W + (size_t)min(n0 + 64 * wn + 32 * j + lr, N - 1) * K + h;
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = v16f_t{};
+        for (int k = s0 * GS_KC; k < s1 * GS_KC; k += 2)
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                const float a = p.A[(size_t)min(m0 + 32 * (2 * i + wm) + lr, M - 1) * K + k + h];
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w[j][k], acc[i][j], 0, 0, 0);
+            }
+    };
+    auto segment = [&](int m0, int n0, int s0, int s1, v16f_t (&acc)[MT][2]) {
+        const uint8_t* const ab = reinterpret_cast<const uint8_t*>(p.A + (size_t)m0 * K);
+        const uint8_t* const wb = reinterpret_cast<const uint8_t*>(p.W + (size_t)n0 * K);
+        uint32_t off[L::NC];
+        static_for<L::NC>([&](auto fc) {
+            constexpr int F = decltype(fc)::value;
+            const int r = F < L::NA ? min(128 * F + cr, M - 1 - m0) : min(128 * (F - L::NA) + cr, N - 1 - n0);
+            off[F] = ((uint32_t)r * (uint32_t)K + 4u * (uint32_t)k4) * 4u;
+        });
+        v4f_t x[L::NC];
+        auto load = [&](auto fc, int s) {
+            constexpr int F = decltype(fc)::value;
+            if (F == L::NA - 1 && !a_last) return;
+            const uint8_t* base = (F < L::NA ? ab : wb) + (size_t)min(s, s1 - 1) * (GS_KC * 4);
+            x[F] = *reinterpret_cast<const v4f_t*>(base + off[F]);
+        };
+        auto put = [&](auto fc, auto bc, int s) {  // split float4 F of stage s into buffer B
+            constexpr int F = decltype(fc)::value, B = decltype(bc)::value;
+            if (F == L::NA - 1 && !a_last) return;
+            if constexpr (F < L::NA) x[F] *= turn_sign<GS_TURN>(s - s0);
+            const Split2 a = split2(x[F][0], x[F][1]), b = split2(x[F][2], x[F][3]);
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                uint8_t* d = F < L::NA ? wr_a + B * L::BYTES + q * L::PIECE_A + F * 2048
+                                       : wr_w + B * L::BYTES + q * L::PIECE_W + (F - L::NA) * 2048;
+                *reinterpret_cast<uint2*>(d) = make_uint2(a.p[q], b.p[q]);
+            }
+        };
+        v4i_t af[2][3], wf[2][2][3];  // [parity][piece], [parity][subtile][piece]
+        auto read_a = [&](auto ic, auto bc, auto pc) {
+            constexpr int I = decltype(ic)::value, B = decltype(bc)::value, P = decltype(pc)::value;
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                af[P][q] = *reinterpret_cast<const v4i_t*>(rd_a + B * L::BYTES + q * L::PIECE_A + I * 1024);
+        };
+        auto read_w = [&](auto bc) {
+            constexpr int B = decltype(bc)::value;
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int q = 0; q < 3; q++)
+                    wf[B][j][q] = *reinterpret_cast<const v4i_t*>(rd_w + B * L::BYTES + q * L::PIECE_W + j * 512);
+        };
+        using C0 = std::integral_constant<int, 0>;
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = v16f_t{};
+        static_for<L::NC>([&](auto fc) { load(fc, s0); });
+        __syncthreads();  // every wave is done with the last segment's stages
+        static_for<L::NC>([&](auto fc) {
+            put(fc, C0{}, s0);
+            load(fc, s0 + 1);
+        });
+        __syncthreads();
+        read_w(C0{});
+        read_a(C0{}, C0{}, C0{});
+        auto stage = [&](auto bc, int s) {
+            constexpr int B = decltype(bc)::value, NB = 1 - B;  // buffer of stage s: s - s0 is even <=> B = 0
+            static_for<MT>([&](auto ic) {
+                constexpr int I = decltype(ic)::value;
+                constexpr int P = (B * MT + I) & 1;  // parity of this group's A operands
+                if constexpr (I == MT - 1) {
+                    __syncthreads();  // stage s + 1 is in LDS, stage s is read out
+                    read_w(std::integral_constant<int, NB>{});
+                    read_a(C0{}, std::integral_constant<int, NB>{}, std::integral_constant<int, 1 - P>{});
+                } else {
+                    read_a(std::integral_constant<int, I + 1>{}, bc, std::integral_constant<int, 1 - P>{});
+                    // this group's share of the next stage
+                    static_for<L::NC>([&](auto fc) {
+                        constexpr int F = decltype(fc)::value;
+                        if constexpr (F * (MT - 1) / L::NC == I) {
+                            put(fc, std::integral_constant<int, NB>{}, s + 1);
+                            load(fc, s + 2);
+                        }
+                    });
+                }
+                // the small products first
+                constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PW[6] = {0, 2, 1, 0, 1, 0};
+                if (I < MT - 1 || mv == MT) {
+#pragma unroll
+                    for (int c = 0; c < 6; c++)
+#pragma unroll
+                        for (int j = 0; j < 2; j++) acc[I][j] = mfma_bf16(af[P][PA[c]], wf[B][j][PW[c]], acc[I][j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // one group's operands and stores at a time
+            });
+        };
+        auto negate = [&] {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = -acc[i][j];
+        };
+        for (int s = s0; s < s1; s += 2) {
+            if (flip_at<GS_TURN>(s - s0)) negate();
+            stage(C0{}, s);
+            if (s + 1 < s1) stage(std::integral_constant<int, 1>{}, s + 1);
+        }
+        if (turn_sign<GS_TURN>(s1 - 1 - s0) < 0.0f) negate();
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) bad |= non_finite(acc[i][j][v]);
+        if (__any(bad)) segment_f32(m0, n0, s0, s1, acc);
+    };
+
+    v16f_t acc[MT][2];
+    auto store = [&](int m0, int n0) {
+        int r0 = m0 + 4 * h;
+        lds_pin(r0);  // the row offsets are formed here, not kept across the stage loop
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            if (i >= mv) break;  // wave-uniform: the next tile's rows
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int col = n0 + 64 * wn + 32 * j + lr;
+                if (col >= N) continue;
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int row = 32 * (2 * i + wm) + 8 * (v / 4) + r0 + v % 4;
+                    if (row >= M) continue;
+                    const size_t o = (size_t)row * N + col;
+                    p.C[o] = p.R ? p.R[o] + acc[i][j][v] : acc[i][j][v];
+                }
+            }
+        }
+    };
+    // an XCD (work groups go round robin over the eight) takes neighbouring ranges
+    const int g = p.G % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (p.G / 8) + (int)blockIdx.x / 8;
+    const int lo = gs_lo(p, g), hi = gs_lo(p, g + 1);
+    for (int u = lo; u < hi;) {
+        const int t = u / nst, s0 = u - t * nst, s1 = min(nst, s0 + (hi - u));
+        int m, n;
+        gs_tile(p, t, m, n);
+        segment(m * p.bm, n * GS_BN, s0, s1, acc);
+        if (s0 == 0 && s1 == nst) {
+            store(m * p.bm, n * GS_BN);
+        } else {
+            float* slot = p.part + (size_t)(2 * g + (u == lo ? 0 : 1)) * (MT * 64 * GS_BN) + tid;
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) slot[((i * 2 + j) * 16 + v) * GS_THREADS] = acc[i][j][v];
+        }
+        u += s1 - s0;
+    }
+}
+
+// Sum of the pieces of every cut tile, in k order (+ R): work group (t, y) takes values
+// 4 y .. 4 y + 3 (value 32 i + 16 j + v) of every thread of tile t.
+template <int MT>
+__global__ __launch_bounds__(GS_THREADS) void gemm_split_sum_kernel(GemmSplitArgs p) {
+    const int nst = p.K / GS_KC;
+    const int t = blockIdx.x;
+    const int u0 = t * nst, u1 = u0 + nst - 1;
+    const int g0 = gs_owner(p, u0), g1 = gs_owner(p, u1);
+    if (g0 == g1) return;
+    const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE, wm = wv / 4, wn = wv % 4;
+    const int lr = lane % 32, h = lane / 32;
+    const int i = blockIdx.y / 8, j = blockIdx.y / 4 % 2;
+    if (2 * i + wm >= p.bm / 32) return;
+    // the first piece is g0's last one unless g0's range starts at this tile
+    const int slot0 = 2 * g0 + (gs_lo(p, g0) == u0 ? 0 : 1);
+    const float* __restrict__ part = p.part + (size_t)blockIdx.y * 4 * GS_THREADS + tid;
+    constexpr size_t SLOT = MT * 64 * GS_BN;
+    float sum[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) sum[v] = part[slot0 * SLOT + v * GS_THREADS];
+    for (int g = g0 + 1; g <= g1; g++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) sum[v] += part[2 * (size_t)g * SLOT + v * GS_THREADS];
+    int m, n;
+    gs_tile(p, t, m, n);
+    const int col = n * GS_BN + 64 * wn + 32 * j + lr;
+    if (col >= p.N) return;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = m * p.bm + 32 * (2 * i + wm) + 8 * (blockIdx.y % 4) + 4 * h + v;
+        if (row >= p.M) break;
+        const size_t o = (size_t)row * p.N + col;
+        p.C[o] = p.R ? p.R[o] + sum[v] : sum[v];
+    }
+}
+
+template <int MT>
+static hipError_t gemm_split_launch(const GemmSplitArgs& p, hipStream_t s) {
+    hipLaunchKernelGGL(gemm_split_kernel<MT>, dim3(p.G), dim3(GS_THREADS), 0, s, p);
+    // ranges that are whole tiles leave no pieces
+    if (p.mt * p.nt % p.G != 0)
+        hipLaunchKernelGGL(gemm_split_sum_kernel<MT>, dim3(p.mt * p.nt, 8 * MT), dim3(GS_THREADS), 0, s, p);
+    return hipGetLastError();
+}
+
+// rows of A per tile: up to 256; half that where whole tiles have to fill the chip and would
+// not twice over
+static int gs_rows(int M, int N, bool ws) {
+    return !ws && (int64_t)((M + 255) / 256) * ((N + GS_BN - 1) / GS_BN) < 2 * GEMM_SPLIT_GROUPS ? 128 : 256;
+}
+
+bool gemm_split_ok(int M, int N, int K, bool ws) {
+    const int rows = gs_rows(M, N, ws);
+    const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + GS_BN - 1) / GS_BN);
+    // 32-bit unit counts and row offsets
+    if (M <= 64 || K % GS_KC != 0 || K > (1 << 20) || tiles * (K / GS_KC) >= (1 << 30)) return false;
+    return ws || tiles >= GEMM_SPLIT_GROUPS;
+}
+
+hipError_t launch_gemm_split(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
+                             hipStream_t s, float* ws) {
+    const int rows = gs_rows(M, N, ws != nullptr);
+    int mt = (M + rows - 1) / rows;
+    const int nt = (N + GS_BN - 1) / GS_BN;
+    const int sub = (M + 32 * mt - 1) / (32 * mt);  // 32-row subtiles of a tile
+    mt = (M + 32 * sub - 1) / (32 * sub);
+    const int tiles = mt * nt, U = tiles * (K / GS_KC);
+    // with scratch: one work group per CU, eight stages each at least
+    const int G = !ws ? tiles : U < 8 * GEMM_SPLIT_GROUPS ? (U + 7) / 8 : GEMM_SPLIT_GROUPS;
+    const GemmSplitArgs p{A, W, R, C, M, N, K, 32 * sub, mt, nt, G, U / G, U % G, ws};
+    switch ((sub + 1) / 2) {
+    case 1:
+    case 2: return gemm_split_launch<2>(p, s);
+    case 3: return gemm_split_launch<3>(p, s);
+    default: return gemm_split_launch<4>(p, s);
+    }
+}
+
+size_t gemm_split_ws_bytes() { return (size_t)2 * GEMM_SPLIT_GROUPS * 256 * GS_BN * 4; }
 
 }  // namespace hy

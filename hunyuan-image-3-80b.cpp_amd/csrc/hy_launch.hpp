@@ -193,9 +193,10 @@ constexpr int FA_SPLIT_SLOTS = 4096;
 int flash_attn_ws_slots(int max_tokens, int max_keys, int nkv);
 size_t flash_attn_ws_floats(int hd, int slots);
 // C = A . W^T, plus R elementwise when R is not null (R may alias nothing written here).
-// ws: gemm_nt_f32_ws_bytes() of device scratch for the stream-K split of mid-size grids
-// (gemm_nt_f32_uses_ws); without it those grids run one tile per work group.
-constexpr int GEMM_SK_GROUPS = 512;  // stream-K work groups: two per CU
+// ws: gemm_nt_f32_ws_bytes() of device scratch for the pieces of tiles that are cut between
+// work groups; without it a work group takes whole tiles.
+constexpr int GEMM_SK_GROUPS = 512;     // work groups of the small-batch product: two per CU
+constexpr int GEMM_SPLIT_GROUPS = 256;  // of the larger one: one per CU
 size_t gemm_nt_f32_ws_bytes();
 bool gemm_nt_f32_uses_ws(int M, int N, int K);
 hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
@@ -205,6 +206,12 @@ hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, fl
 bool gemm_small_ok(int M, int N, int K);
 hipError_t launch_gemm_small(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                              hipStream_t s, float* ws);
+// and for more rows (hy_gemm.hip), K a multiple of 16; without ws only where whole tiles
+// fill the chip
+bool gemm_split_ok(int M, int N, int K, bool ws);
+hipError_t launch_gemm_split(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
+                             hipStream_t s, float* ws);
+size_t gemm_split_ws_bytes();
 hipError_t launch_rope_qknorm(const RopeNormArgs& a, hipStream_t s);
 // ws: flash_attn_ws_floats(hd, ws_slots) of device scratch, or nullptr (no split over
 // the keys)
