@@ -5,24 +5,16 @@
 // 2D rotary tables (src/hunyuan_image_gen.cpp:11-117).
 //
 // Kernels:
-//  * gemm_nt_f32_lds_kernel / gemm_nt_f32_kernel: C[M][N] = (R[M][N] +) A[M][K] .
-//    W[N][K]^T on v_mfma_f32_32x32x2f32 (the QKV and output projections; R is the
-//    decoder layer's residual stream when the output projection adds it).  Waves of
-//    64 x 64 (2 x 2 MFMA tiles).  Large grids: four waves per 128 x 128 work group,
-//    K in stages of 32 (16) floats DMA-copied into a swizzled LDS ring.  Mid-size
-//    grids (64..1023 tiles): the same kernel as 512 stream-K work groups that split
-//    the tiles' K stages evenly, and gemm_fixup_kernel summing the cut tiles' pieces
-//    in K order.  17 to 128 rows of A with K % 32 == 0: hy_gemm.hip.  Other small
-//    grids: one wave per work group, K in steps of 16 straight from global memory into
-//    registers.
+//  * launch_gemm_nt_f32: C[M][N] = (R[M][N] +) A[M][K] . W[N][K]^T (the QKV and output
+//    projections; R is the decoder layer's residual stream when the output projection
+//    adds it).  Up to 16 rows of A: gemv_nt_f32_kernel; more: hy_gemm.hip; the few grids
+//    that one does not take: gemm_nt_f32_kernel, one wave per 64 x 64 tile on
+//    v_mfma_f32_32x32x2f32, K in steps of 16 straight from global memory into registers.
 //  * rope_qknorm_kernel: one wave per (token, head): rotary embedding (1D positions,
 //    2D tables or none), per-head RMSNorm, written to q [T][nh][hd] and, for key
 //    heads, k / v into a [nkv][L][hd] cache at row pos0 + t.
-//  * flash_attn_kernel<HD>: one work group per (32-query tile, kv group), one wave
-//    per query head of the group (4 heads share the group's K / V blocks in LDS).
-//    Scores are computed transposed, S^T = K Q^T (keys on MFMA rows, queries on the
-//    lanes), so a query's online-softmax statistics stay in its lane pair; P^T then
-//    feeds O^T += V^T P^T straight from the score registers.
+//  * flash_merge_kernel, flash_decode16_kernel, flash_decode_kernel: the prompt
+//    attention's (hy_flash.hip) join over key chunks, and attention of up to 8 queries.
 //
 // fp32 MFMA layouts (v_mfma_f32_32x32x2f32, checked on the device): A lane l holds
 // A[l%32][l/32], B lane l holds B[l/32][l%32], result register v of lane l is
@@ -190,7 +182,9 @@ __global__ __launch_bounds__(256) void gemv_nt_f32_kernel(const float* __restric
     }
 }
 
-size_t gemm_nt_f32_ws_bytes() { return gemm_split_ws_bytes(); }
+size_t gemm_nt_f32_ws_bytes(int max_rows) {
+    return max(gemm_small_ws_bytes(max_rows), gemm_split_ws_bytes(max_rows));
+}
 
 // the grids of the stand-alone product that are given scratch: 64 to 1023 tiles of 128 x 128
 bool gemm_nt_f32_uses_ws(int M, int N, int K) {
@@ -348,217 +342,8 @@ hipError_t launch_rope2d_table(int seq, int n_elem, int text_len, int img_h, int
 }
 
 // ---------------------------------------------------------------- flash attention
-// LDS row pitches (floats): K rows are read 16 B per lane by 32 rows (pitch = 4 mod
-// 64 banks: 16 consecutive rows hit 16 distinct bank quads); V rows 4 B per lane by
-// two rows 4 apart per instruction (pitch = 8 mod 16: the two half-waves land on
-// opposite bank halves).
-// K / V blocks of 32 keys reach LDS by DMA (global_load_lds_dwordx4) into a 2-deep
-// ring: the next block's copies are in flight during a block's math, no registers
-// hold them, and one barrier per block suffices.  Rows are HD floats (HD / 4 16-byte
-// chunks), unpadded; chunk c of K row r sits at position c ^ (r & 15) and chunk c of V
-// row r at c ^ 8 ((r >> 2) & 1).  Then the K reads of 16 consecutive rows at one
-// logical chunk (QK^T) and the V reads of rows key and key + 4 by the two half-waves
-// (PV) fall on distinct bank groups.  Each lane of a copy fetches the chunk that
-// belongs at its position.
-template <int HD>
-struct FaShape {
-    static constexpr int ROWB = HD * 4;         // bytes per row
-    static constexpr int BLK = 32 * ROWB;       // one K (or V) block
-    static constexpr int BUF = 2 * BLK;         // K block, then V block
-    static constexpr int CPW = BLK / 1024 / 4;  // 1 KB copies per wave for K (and for V)
-    static constexpr int RPC = 1024 / ROWB;     // rows per copy
-    static_assert(CPW >= 1 && HD / 4 >= 16, "head_dim 64 or 128");
-};
-__device__ __forceinline__ int fa_swz_k(int r) { return r & 15; }
-__device__ __forceinline__ int fa_swz_v(int r) { return 8 * ((r >> 2) & 1); }
-
-template <int HD>
-__global__ __launch_bounds__(256, 2) void flash_attn_kernel(FlashArgs a) {
-    using S = FaShape<HD>;
-    __shared__ __attribute__((aligned(1024))) uint8_t ring[2][S::BUF];
-    const int tid = threadIdx.x, lane = tid % WAVE;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    const int lr = lane % 32, h = lane / 32;
-    const int n_qt = (a.T + 31) / 32;
-    // chunk-major, and inside a chunk the longest (causal) query tiles first
-    const int per_chunk = n_qt * a.nkv;
-    const int chunk = (int)blockIdx.x / per_chunk, rem = (int)blockIdx.x % per_chunk;
-    const int qt = n_qt - 1 - rem / a.nkv;
-    const int g = rem % a.nkv;
-    const int q0 = qt * 32;
-    const int head = g * 4 + wave;  // 4 query heads per kv group
-    const int qrow = min(q0 + lr, a.T - 1);
-
-    // visible keys: all kv_len, or (causal) keys <= q_pos0 + q
-    const int last_q = min(q0 + 31, a.T - 1);
-    const int key_end = a.causal ? min(a.kv_len, a.q_pos0 + last_q + 1) : a.kv_len;
-    const int nblk = (key_end + 31) / 32;
-    // this work group's key blocks: all of them, or chunk `chunk` of cb blocks
-    const int nc = a.cb ? (nblk + a.cb - 1) / a.cb : 1;
-    if (chunk >= nc) return;  // whole work group: the tile has fewer chunks
-    const int kb0 = a.cb ? chunk * a.cb : 0, kb1 = a.cb ? min(nblk, kb0 + a.cb) : nblk;
-
-    // copies: copy q of this wave moves rows (wave CPW + q) RPC .. + RPC - 1 of the
-    // block; lane l lands at byte 16 l of it: row + l / (ROWB / 16), position
-    // l % (ROWB / 16), fetching the chunk stored there
-    const float* kg = a.k + (size_t)g * a.L * HD;
-    const float* vg = a.v + (size_t)g * a.L * HD;
-    int crow[S::CPW], kchunk[S::CPW], vchunk[S::CPW];
-#pragma unroll
-    for (int q = 0; q < S::CPW; q++) {
-        crow[q] = (wave * S::CPW + q) * S::RPC + lane / (S::ROWB / 16);
-        const int pos = lane % (S::ROWB / 16);
-        kchunk[q] = 4 * (pos ^ fa_swz_k(crow[q]));
-        vchunk[q] = 4 * (pos ^ fa_swz_v(crow[q]));
-    }
-    auto issue = [&](int kb) {
-        uint8_t* buf = ring[(kb - kb0) & 1];
-#pragma unroll
-        for (int q = 0; q < S::CPW; q++) {
-            const size_t row = (size_t)min(kb * 32 + crow[q], a.kv_len - 1) * HD;  // in bounds
-            g2l16(kg + row + kchunk[q], buf + (wave * S::CPW + q) * 1024);
-            g2l16(vg + row + vchunk[q], buf + S::BLK + (wave * S::CPW + q) * 1024);
-        }
-    };
-    issue(kb0);
-
-    // Q resident: lane (query lr, half h) holds Q[q][16c + 8h + j], pre-multiplied by
-    // scale * log2(e): the scores come out in the base-2 domain, where the softmax uses
-    // the hardware 2^x (v_exp_f32; 2^-inf = 0 serves the masked keys)
-    const float qscale = a.scale * 1.4426950408889634f;
-    float qv[HD / 2];
-    {
-        const float* qp = a.q + ((size_t)qrow * a.nh + head) * HD + 8 * h;
-#pragma unroll
-        for (int c = 0; c < HD / 16; c++) {
-            const v4f_t x0 = *reinterpret_cast<const v4f_t*>(qp + 16 * c);
-            const v4f_t x1 = *reinterpret_cast<const v4f_t*>(qp + 16 * c + 4);
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                qv[8 * c + j] = x0[j] * qscale;
-                qv[8 * c + 4 + j] = x1[j] * qscale;
-            }
-        }
-    }
-    // LDS read offsets inside a buffer: K row lr at logical chunk 4c + 2h + t; V rows
-    // 8 i + 4 h + j at float 32 c + lr (the row part 8 i + j is an immediate)
-    const int swk = fa_swz_k(lr);
-    uint32_t voff[HD / 32];
-#pragma unroll
-    for (int c = 0; c < HD / 32; c++) voff[c] = (uint32_t)(S::BLK + 4 * h * S::ROWB + 128 * (c ^ h) + 4 * lr);
-    const uint32_t ring0 = lds_off(ring[0]);
-
-    v16f_t o[HD / 32];
-#pragma unroll
-    for (int c = 0; c < HD / 32; c++) o[c] = v16f_t{};
-    float m_run = -INFINITY, l_run = 0.0f;
-    const int my_q = a.q_pos0 + q0 + lr;  // key index of this lane's query (causal bound)
-
-    for (int kb = kb0; kb < kb1; kb++) {
-        MM_WAIT_VM_LGKM(0);  // this wave's copies of block kb have landed
-        __syncthreads();     // everyone's have, and block kb - 1's buffer is free
-        if (kb + 1 < kb1) issue(kb + 1);
-        const uint32_t base = ring0 + (uint32_t)(((kb - kb0) & 1) * S::BUF);
-        // S^T[key][q] = sum_d K[key][d] Q[q][d]: all K reads of the block in flight,
-        // consumed in order
-        const uint32_t krow = base + (uint32_t)(lr * S::ROWB);
-        v4i_t kr[HD / 16][2];
-#pragma unroll
-        for (int c = 0; c < HD / 16; c++)
-#pragma unroll
-            for (int t = 0; t < 2; t++) kr[c][t] = lds_b128_at<0>(krow + 16u * (uint32_t)((4 * c + 2 * h + t) ^ swk));
-        v16f_t s = v16f_t{};
-        [&]<int... C>(std::integer_sequence<int, C...>) {
-            (
-                [&] {
-                    lds_wait_upto<HD / 8 - 2 - 2 * C>();
-                    lds_pin(kr[C][0]);
-                    lds_pin(kr[C][1]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++)
-                        s = mfma_f32(__int_as_float(kr[C][j / 4][j % 4]), qv[8 * C + j], s);
-                }(),
-                ...);
-        }(std::make_integer_sequence<int, HD / 16>{});
-        // mask (only blocks that reach past the tile's first query or past kv_len),
-        // online softmax over this lane pair's 32 keys
-        const bool need_mask = kb * 32 + 31 >= a.kv_len || (a.causal && kb * 32 + 31 > a.q_pos0 + q0);
-        if (need_mask) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int key = kb * 32 + 8 * (v / 4) + 4 * h + v % 4;
-                if (key >= a.kv_len || (a.causal && key > my_q)) s[v] = -INFINITY;
-            }
-        }
-        float mloc = s[0];
-#pragma unroll
-        for (int v = 1; v < 16; v++) mloc = fmaxf(mloc, s[v]);
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, WAVE));
-        // every processed block leaves at least one visible key per query, so m_new is
-        // finite
-        const float m_new = fmaxf(m_run, mloc);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 for the first block
-        float psum = 0.0f;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const float p = __builtin_amdgcn_exp2f(s[v] - m_new);
-            s[v] = p;
-            psum += p;
-        }
-        psum += __shfl_xor(psum, 32, WAVE);
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        if (__ballot(alpha != 1.0f)) {  // the running max moved for some query
-#pragma unroll
-            for (int c = 0; c < HD / 32; c++) o[c] *= alpha;
-        }
-        // O^T[d][q] += sum_key V[key][d] P^T[key][q]: per 32 dims, the 16 key values
-        // of the lane in two groups of 8 reads
-#pragma unroll
-        for (int c = 0; c < HD / 32; c++) {
-            const uint32_t vb = base + voff[c];
-            uint32_t vv[16];
-            [&]<int... V>(std::integer_sequence<int, V...>) {
-                ((vv[V] = lds_b32_at<(8 * (V / 4) + V % 4) * S::ROWB>(vb)), ...);
-            }(std::make_integer_sequence<int, 16>{});
-            lds_wait_upto<8>();
-#pragma unroll
-            for (int v = 0; v < 8; v++) {
-                lds_pin(vv[v]);
-                o[c] = mfma_f32(__uint_as_float(vv[v]), s[v], o[c]);
-            }
-            lds_wait_upto<0>();
-#pragma unroll
-            for (int v = 8; v < 16; v++) {
-                lds_pin(vv[v]);
-                o[c] = mfma_f32(__uint_as_float(vv[v]), s[v], o[c]);
-            }
-        }
-    }
-    if (nc > 1) {
-        // partial result of this chunk: unnormalised O^T, running max and sum
-        float* pp = a.part + ((size_t)((qt * a.nch + chunk) * a.nkv + g) * 4 + wave) * (HD * 32 + 128);
-#pragma unroll
-        for (int c = 0; c < HD / 32; c++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) pp[(c * 16 + v) * 64 + lane] = o[c][v];
-        pp[HD * 32 + lane] = m_run;
-        pp[HD * 32 + 64 + lane] = l_run;
-        return;
-    }
-    if (q0 + lr >= a.T) return;
-    const float inv = 1.0f / l_run;
-    float* op = a.out + ((size_t)(q0 + lr) * a.nh + head) * HD;
-#pragma unroll
-    for (int c = 0; c < HD / 32; c++)
-#pragma unroll
-        for (int v4 = 0; v4 < 4; v4++) {
-            const int d = 32 * c + 8 * v4 + 4 * h;
-            *reinterpret_cast<float4*>(op + d) = make_float4(o[c][4 * v4] * inv, o[c][4 * v4 + 1] * inv,
-                                                             o[c][4 * v4 + 2] * inv, o[c][4 * v4 + 3] * inv);
-        }
-}
-
+// The prompt's attention is hy_flash.hip; here its join over key chunks, the decode kernels
+// and the launch.
 // Join the chunks of every split query tile: work group (tile x kv group, piece y)
 // takes 4 of the output values of every thread of the attention kernel's layout
 // (y = 4 cc + v4: dims 32 cc + 8 v4 + 4 h .. + 3 of query lr).  With M = max_c m_c,
@@ -610,6 +395,23 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a) {
 // DMA, in the prompt kernel's swizzled layout, read by the same MFMA steps.  The wave
 // writes unnormalised O, running max and sum of its 4T live rows;
 // flash_decode_merge_kernel joins the waves of a group.
+// K / V blocks of 32 keys reach LDS by DMA.  Rows are HD floats (HD / 4 16-byte chunks),
+// unpadded; chunk c of K row r sits at position c ^ (r & 15) and chunk c of V row r at
+// c ^ 8 ((r >> 2) & 1).  Then the K reads of 16 consecutive rows at one logical chunk
+// (QK^T) and the V reads of rows key and key + 4 by the two half-waves (PV) fall on
+// distinct bank groups.  Each lane of a copy fetches the chunk that belongs at its
+// position.
+template <int HD>
+struct FaShape {
+    static constexpr int ROWB = HD * 4;      // bytes per row
+    static constexpr int BLK = 32 * ROWB;    // one K (or V) block
+    static constexpr int BUF = 2 * BLK;      // K block, then V block
+    static constexpr int RPC = 1024 / ROWB;  // rows per copy
+    static_assert(HD / 4 >= 16, "head_dim 64 or 128");
+};
+__device__ __forceinline__ int fa_swz_k(int r) { return r & 15; }
+__device__ __forceinline__ int fa_swz_v(int r) { return 8 * ((r >> 2) & 1); }
+
 template <int HD>
 __global__ __launch_bounds__(64) void flash_decode_kernel(FlashArgs a) {
     using S = FaShape<HD>;
@@ -1006,13 +808,13 @@ hipError_t launch_flash_attn(const FlashArgs& a_in, hipStream_t s, float* ws, in
     a.cb = 0;
     a.nch = 1;
     // Split the keys of each query tile into chunks of cb blocks when that shortens the
-    // launch.  Cost model, in units of one key block of one work group (~6.8 us at two
-    // work groups per CU):
+    // launch.  Cost model, in units of one key block of one work group (~4 us at head_dim
+    // 128):
     //   whole tiles (longest first):  max(longest tile, all blocks / resident groups) + 1
-    //   chunks of cb:                 rounds x (cb + 1) + partial-tile traffic
-    // (+1: the ramp of a round; the partials are written and read back by the merge at
-    // ~5 TB/s, ~34 MB per unit of time).  Short prompts, causal tiles of very different
-    // lengths and decode against a long cache split; long prompts fill the chip with
+    //   chunks of cb:                 rounds x (cb + 1) + partial-tile traffic + 1.5
+    // (+1: the ramp of a round; 1.5: the merge's launch; the partials are written and read back by the merge at
+    // ~5 TB/s, ~20 MB per unit of time).  Short prompts, causal tiles of very different
+    // lengths and a few queries against a long cache split; long prompts fill the chip with
     // whole tiles.
     if (a.T <= 8 && ws && max_nblk >= 2) {
         // decode: one wave per cb key blocks of a group, at most half as many waves as
@@ -1054,25 +856,26 @@ hipError_t launch_flash_attn(const FlashArgs& a_in, hipStream_t s, float* ws, in
         }
         return hipGetLastError();
     }
-    const int slots = 256 * (a.hd == 128 ? 2 : 3);  // resident work groups (occupancy)
+    constexpr int slots = 256;  // resident work groups: one per CU
     if (ws && max_nblk >= 2) {
+        const int n_wt = (a.T + 63) / 64;  // tiles of two 32-query halves
         auto tile_blocks = [&](int t) {
-            const int kend = a.causal ? min(a.kv_len, a.q_pos0 + min(32 * t + 31, a.T - 1) + 1) : a.kv_len;
+            const int kend = a.causal ? min(a.kv_len, a.q_pos0 + min(64 * t + 63, a.T - 1) + 1) : a.kv_len;
             return (kend + 31) / 32;
         };
         long total = 0;
-        for (int t = 0; t < n_qt; t++) total += tile_blocks(t);
+        for (int t = 0; t < n_wt; t++) total += tile_blocks(t);
         total *= a.nkv;
-        const double part_units = 2.0 * 4 * (a.hd * 32 + 128) * 4 / 34e6;  // per split unit
+        const double part_units = 2.0 * 8 * (128 * 32 + 128) * 4 / 20e6;  // per split unit
         double best = (double)max((long)max_nblk, (total + slots - 1) / slots) + 1;
         int best_cb = 0;
         for (int cb = 1; cb < max_nblk; cb++) {
             const int nch = (max_nblk + cb - 1) / cb;
             if ((long)n_qt * nch * a.nkv > ws_slots) continue;
             long units = 0;
-            for (int t = 0; t < n_qt; t++) units += (tile_blocks(t) + cb - 1) / cb;
+            for (int t = 0; t < n_wt; t++) units += (tile_blocks(t) + cb - 1) / cb;
             units *= a.nkv;
-            const double cost = (double)((units + slots - 1) / slots) * (cb + 1) + units * part_units;
+            const double cost = (double)((units + slots - 1) / slots) * (cb + 1) + units * part_units + 1.5;
             if (cost < best) {
                 best = cost;
                 best_cb = cb;
@@ -1084,14 +887,7 @@ hipError_t launch_flash_attn(const FlashArgs& a_in, hipStream_t s, float* ws, in
             a.part = ws;
         }
     }
-    const dim3 grid((unsigned)(base * a.nch));
-    if (a.hd == 128)
-        hipLaunchKernelGGL(flash_attn_kernel<128>, grid, dim3(256), 0, s, a);
-    else if (a.hd == 64)
-        hipLaunchKernelGGL(flash_attn_kernel<64>, grid, dim3(256), 0, s, a);
-    else
-        return hipErrorInvalidValue;
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch_flash_split(a, s);
     if (e != hipSuccess || !a.cb) return e;
     if (a.hd == 128)
         hipLaunchKernelGGL(flash_merge_kernel<128>, dim3((unsigned)base, 128 / 8), dim3(256), 0, s, a);

@@ -268,7 +268,7 @@ int hy_attn_create(const hy_attn_config* cfg, hy_attn_ctx** out) {
         size_t n;
     } parts[] = {{&c->qkv, Tm * c->nqkv}, {&c->q, Tm * nq},  {&c->kf, Tm * nk},   {&c->vf, Tm * nk},
                  {&c->merged, Tm * nq},   {&c->xn, Tm * H}, {&c->hres, Tm * H},
-                 {&c->gemm_ws, hy::gemm_nt_f32_ws_bytes() / 4},
+                 {&c->gemm_ws, hy::gemm_nt_f32_ws_bytes(c->Tm) / 4},
                  {&c->fa_ws, hy::flash_attn_ws_floats(c->hd, c->fa_slots)}};
     size_t total = 0;
     for (auto& p : parts) total += al256(p.n * 4);
@@ -486,7 +486,7 @@ int hy_lm_head_f32(const float* x, const float* w, const float* resid, uint32_t 
         hipEvent_t ev = nullptr;
         HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         float* ws = nullptr;
-        if (hipMalloc(reinterpret_cast<void**>(&ws), hy::gemm_nt_f32_ws_bytes()) != hipSuccess) {
+        if (hipMalloc(reinterpret_cast<void**>(&ws), hy::gemm_nt_f32_ws_bytes(1 << 20)) != hipSuccess) {
             (void)hipEventDestroy(ev);
             return fail(HY_ERR_NOMEM, "GEMM scratch allocation failed");
         }

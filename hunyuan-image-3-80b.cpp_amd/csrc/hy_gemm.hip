@@ -1,82 +1,19 @@
 // hy_gemm.hip -- fp32 matrix products C[M][N] = (R[M][N] +) A[M][K] . W[N][K]^T on the
 // bf16 matrix cores, with fp32 accuracy.
 //
-// Every fp32 operand is split exactly into three bf16 pieces, x = hi + mid + lo (8 + 8 + 8
-// significand bits, round to nearest at each step, both remainders exact in fp32; bf16
-// has fp32's exponent range and the matrix cores keep bf16 denormals), and a product is
-// the sum of the six piece products of weight 2^-16 and above,
-//   hi hi + hi mid + mid hi + mid mid + hi lo + lo hi,
-// accumulated in fp32 by v_mfma_f32_32x32x16_bf16.  What is left out, mid lo + lo mid +
-// lo lo, is below 2^-24 of the product: no more than one fp32 rounding of it.  Six
-// bf16 MFMAs of 16 k-steps take 6 x 32 cycles where eight fp32 MFMAs of 2 take 8 x 64.
-//
-// These instructions cut the low bits of what they add towards minus infinity (measured: a
-// mean error of -0.21 of the rms error, whatever the result's sign; the fp32 MFMAs show
-// none), and a later average over rows, as in attention, keeps such a mean while it thins
-// out the rest.  So the accumulators hold the sum and its negative in turns (flip_at),
-// with the pieces of A negated alike, and the mean cancels.
-//
-// The split is exact down to 2^-110; below that the last pieces run out of exponent, an
-// absolute error of at most 2^-134 of the operand.
+// Operands are split into three bf16 pieces each and the six significant piece products
+// summed, with the accumulators' sign in turns: hy_split.hpp.
 //
 // Infinities and NaNs have no such split (inf - inf), and a value that rounds up to
 // infinity in bf16 neither: a wave whose accumulators hold a non-finite value after its
 // k-range computes that range again on the fp32 matrix cores (segment_f32), so such
 // inputs give what the fp32 product gives.
-#include <utility>
-
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
 #include "hy_lds.hpp"
+#include "hy_split.hpp"
 
 namespace hy {
-
-// f(integral_constant 0), ..., f(integral_constant N - 1): loops whose index is a constant
-// (LDS offsets in instructions, register arrays)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-        (f(std::integral_constant<int, I>{}), ...);
-    }(std::make_integer_sequence<int, N>{});
-}
-
-typedef float v16f_t __attribute__((ext_vector_type(16)));
-typedef float v2f_t __attribute__((ext_vector_type(2)));
-typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
-
-// two floats -> their three bf16 pieces, packed (v_cvt_pk_bf16_f32, round to nearest even)
-struct Split2 {
-    uint32_t p[3];
-};
-__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
-    const v2f_t f = {a, b};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, v2bf_t));
-}
-__device__ __forceinline__ Split2 split2(float a, float b) {
-    Split2 s;
-    s.p[0] = pk_bf16(a, b);
-    a -= __uint_as_float(s.p[0] << 16);
-    b -= __uint_as_float(s.p[0] & 0xffff0000u);
-    s.p[1] = pk_bf16(a, b);
-    a -= __uint_as_float(s.p[1] << 16);
-    b -= __uint_as_float(s.p[1] & 0xffff0000u);
-    s.p[2] = pk_bf16(a, b);
-    return s;
-}
-__device__ __forceinline__ v16f_t mfma_bf16(v4i_t a, v4i_t b, v16f_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0,
-                                                   0, 0);
-}
-// Sign turns: PERIOD stages of one sign, the first one half as long, so that the growing
-// means of neighbouring turns cancel.  flip_at: stage d of a range opens a turn;
-// turn_sign: its sign.
-template <int PERIOD>
-__device__ __forceinline__ bool flip_at(int d) { return d % PERIOD == PERIOD / 2; }
-template <int PERIOD>
-__device__ __forceinline__ float turn_sign(int d) { return (d + PERIOD / 2) / PERIOD % 2 ? -1.0f : 1.0f; }
-// finite iff x - x == 0
-__device__ __forceinline__ bool non_finite(float x) { return !(x - x == 0.0f); }
 
 // ---------------------------------------------------------------- small batches (M <= 128)
 // A stream over W: a work group of four waves takes all M rows of A (MT tiles of 32) times
@@ -318,6 +255,10 @@ __global__ __launch_bounds__(256) void gemm_small_sum_kernel(GemmSmallArgs p) {
 bool gemm_small_ok(int M, int N, int K) {
     // 32-bit unit counts
     return M > 16 && M <= 128 && K % SK_KC == 0 && (int64_t)(N + SK_BN) / SK_BN * (K / SK_KC) < (1 << 30);
+}
+
+size_t gemm_small_ws_bytes(int max_rows) {
+    return max_rows <= 16 ? 0 : (size_t)2 * GEMM_SK_GROUPS * (32 * min((max_rows + 31) / 32, 4)) * SK_BN * 4;
 }
 
 template <int MT>
@@ -672,6 +613,10 @@ hipError_t launch_gemm_split(const float* A, const float* W, const float* R, flo
     }
 }
 
-size_t gemm_split_ws_bytes() { return (size_t)2 * GEMM_SPLIT_GROUPS * 256 * GS_BN * 4; }
+size_t gemm_split_ws_bytes(int max_rows) {
+    // slots of 64 MT rows, MT pairs of 32-row subtiles (launch_gemm_split)
+    const int mt = max_rows <= 64 ? 0 : max_rows > 192 ? 4 : max_rows > 128 ? 3 : 2;
+    return (size_t)2 * GEMM_SPLIT_GROUPS * (64 * mt) * GS_BN * 4;
+}
 
 }  // namespace hy

@@ -186,6 +186,8 @@ struct FlashArgs {
     float* part = nullptr;
     int cb = 0, nch = 1;
 };
+// attention of more than 8 queries, chunks as set in the arguments (hy_flash.hip)
+hipError_t launch_flash_split(const FlashArgs& a, hipStream_t s);
 // scratch of the split attention: partial tiles (at most FA_SPLIT_SLOTS) for head_dim
 // hd; flash_attn_ws_slots: the slots a context of max_tokens queries and max_keys
 // keys can use
@@ -193,11 +195,11 @@ constexpr int FA_SPLIT_SLOTS = 4096;
 int flash_attn_ws_slots(int max_tokens, int max_keys, int nkv);
 size_t flash_attn_ws_floats(int hd, int slots);
 // C = A . W^T, plus R elementwise when R is not null (R may alias nothing written here).
-// ws: gemm_nt_f32_ws_bytes() of device scratch for the pieces of tiles that are cut between
+// ws: gemm_nt_f32_ws_bytes(rows of A at most) of device scratch for the pieces of tiles that are cut between
 // work groups; without it a work group takes whole tiles.
 constexpr int GEMM_SK_GROUPS = 512;     // work groups of the small-batch product: two per CU
 constexpr int GEMM_SPLIT_GROUPS = 256;  // of the larger one: one per CU
-size_t gemm_nt_f32_ws_bytes();
+size_t gemm_nt_f32_ws_bytes(int max_rows);
 bool gemm_nt_f32_uses_ws(int M, int N, int K);
 hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                               hipStream_t s, float* ws = nullptr);
@@ -211,7 +213,8 @@ hipError_t launch_gemm_small(const float* A, const float* W, const float* R, flo
 bool gemm_split_ok(int M, int N, int K, bool ws);
 hipError_t launch_gemm_split(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                              hipStream_t s, float* ws);
-size_t gemm_split_ws_bytes();
+size_t gemm_small_ws_bytes(int max_rows);
+size_t gemm_split_ws_bytes(int max_rows);
 hipError_t launch_rope_qknorm(const RopeNormArgs& a, hipStream_t s);
 // ws: flash_attn_ws_floats(hd, ws_slots) of device scratch, or nullptr (no split over
 // the keys)

@@ -307,3 +307,54 @@ def test_gemm_stream_k_scratch_across_streams(gpu):
         check(ob[i].numpy(), xs[i].astype(np.float64) @ w.astype(np.float64).T, f"stream {i}")
     for s in streams:
         s.close()
+
+
+@pytest.mark.parametrize("shp", SHAPES, ids=["hd64", "hd128"])
+@pytest.mark.parametrize("T", [9, 31, 33, 63, 64, 65, 97, 300])
+def test_prompt_tiles(gpu, shp, T):
+    """Edges of the prompt attention's tiles (64 queries in two halves, 32 keys a block) and
+    of the chunks they are cut into, against float64 attention of the device's own q / k /
+    v: causal, and (through a cache) every token seeing every other.  Bound: the two
+    products' and the softmax's fp32 roundings (2^-24 each, some hundred in a chain, partly
+    cancelling) stay below 1e-5 of the result's norm."""
+    m, w = _ctx(gpu, shp, max_tokens=T, max_cache=T, seed=T)
+    nh, nkv, hd = shp["nh"], shp["nkv"], shp["hd"]
+    x = np.random.default_rng(T).standard_normal((T, shp["H"])).astype(np.float32)
+    out, dq, dk, dv = m.run(x, debug=True)
+    q, k, v = dq.reshape(T, nh, hd), dk.reshape(T, nkv, hd), dv.reshape(T, nkv, hd)
+    ref = _attn64(q, k, v, nh, nkv) @ w.o_w.astype(np.float64).T
+    assert np.linalg.norm(out - ref) <= 1e-5 * np.linalg.norm(ref)
+    cache = A.KVCache(nkv, hd, max_len=T)
+    xb, ob = gpu.Buf.from_array(x), gpu.Buf.empty((T, shp["H"]))
+    m.forward_cached(xb, T, ob)
+    check(ob.numpy(), A.attention_cached(w, x, cache), f"cached T={T}")
+    m.close()
+
+
+def test_prompt_values_without_a_split(gpu):
+    """Values whose nearest bf16 is infinity are finite in fp32 and in the output; an
+    infinite value makes the outputs that see it infinite, those before its key block not."""
+    shp = SHAPES[1]
+    T, nh, nkv, hd = 80, shp["nh"], shp["nkv"], shp["hd"]
+    m, w = _ctx(gpu, shp, max_tokens=T, seed=3)
+    nq, nk = nh * hd, nkv * hd
+    qkv = w.qkv_w.copy()
+    qkv[:, 0] = 0.0
+    qkv[nq + nk + 5, :] = 0.0
+    qkv[nq + nk + 5, 0] = 1.0  # dim 5 of the first value head is x[:, 0] itself
+    o_w = (w.o_w * np.float32(2.0 ** -20)).astype(np.float32)
+    m.upload(qkv, o_w, w.q_norm, w.k_norm)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((T, shp["H"])).astype(np.float32)
+    x[40, 0] = np.float32(3.4e38)
+    out, dq, dk, dv = m.run(x, debug=True)
+    q, k, v = dq.reshape(T, nh, hd), dk.reshape(T, nkv, hd), dv.reshape(T, nkv, hd)
+    assert v[40, 0, 5] == np.float32(3.4e38)
+    ref = _attn64(q, k, v, nh, nkv) @ o_w.astype(np.float64).T
+    assert np.isfinite(out).all()
+    for rows in (slice(0, 40), slice(40, T)):
+        assert np.linalg.norm(out[rows] / 2.0 ** 64 - ref[rows] / 2.0 ** 64) <= 1e-5 * np.linalg.norm(ref[rows] / 2.0 ** 64)
+    x[40, 0] = np.inf
+    out = m.run(x)
+    assert np.isfinite(out[:32]).all() and not np.isfinite(out[40:]).any()
+    m.close()
