@@ -198,14 +198,13 @@ int renorm_rule(int32_t norm, uint32_t K) { return (norm == HY_NORM_ALWAYS || (n
 constexpr uint32_t kGemvMaxTokens = 16;
 
 // AUTO mode: the decode GEMV or the MFMA grouped GEMM.  Measured crossover on one MI355X
-// (H 4096, I 3072, E 64, K 8, layer steps over rotating weight sets): Q4_0 GEMV 374 vs
-// MFMA 423 us at T=32, 515 vs 478 at T=48 (up to ~5 pairs per expert); Q8_0 452 vs 464
-// us at T=20, 512 vs 474 at T=24 (up to ~2.5 pairs per expert).
+// (H 4096, I 3072, E 64, K 8): Q4_0 GEMV 304 vs MFMA 318 us at T=24, 361 vs 314 at T=32 (up
+// to ~3 pairs per expert); Q8_0 400 vs 405 us at T=16, 470 vs 426 at T=24 (~2).
 bool gemv_batch(int wt, uint32_t T, int K, int E) {
     if (T <= kGemvMaxTokens) return true;
     const uint64_t pairs = (uint64_t)T * (uint64_t)K;
-    if (wt == HY_TYPE_Q4_0) return pairs <= 5ull * (uint64_t)E;
-    if (wt == HY_TYPE_Q8_0) return 2 * pairs <= 5ull * (uint64_t)E;
+    if (wt == HY_TYPE_Q4_0) return pairs <= 3ull * (uint64_t)E;
+    if (wt == HY_TYPE_Q8_0) return pairs <= 2ull * (uint64_t)E;
     return false;
 }
 

@@ -16,6 +16,7 @@
 //   tall  (ROWS 256, TOK  64, KB 2): eight waves, 4 row slabs x 2 token halves, each
 //         wave 2 x 1 tiles, a 3-stage ring, two work groups per CU -- keeps the waves
 //         busy when experts see ~64 pairs.
+// Fewer pairs per expert: hy_mfma_few.hip.
 // Every wave owns 2 (or 2 x 2) output tiles of 32 rows x 32 tokens and, per 32-wide
 // block and 32 tokens, issues
 // v_mfma_i32_32x32x32_i8: K = 32 is exactly one GGUF block, so each MFMA result is the
@@ -45,12 +46,9 @@
 #include "hy_launch.hpp"
 #include "hy_layout.hpp"
 #include "hy_lds.hpp"
+#include "hy_mfma.hpp"
 
 namespace hy {
-
-typedef int v16i_t __attribute__((ext_vector_type(16)));
-typedef float v16f_t __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 
 constexpr int MM_XCD = 8;                  // XCDs of the device (work-group round robin)
 constexpr int MM_CU_PER_XCD = 32;          // CUs per XCD (256 in all)
@@ -101,23 +99,6 @@ struct MmShape {
 using ShapeWide = MmShape<128, 128, 2, 4, 2, 2, 4>;
 using ShapeTall = MmShape<256, 64, 2>;
 
-struct MmArgs {
-    MatView W;
-    Routing R;
-    const int8_t* aq;   // activations int8, block-major in slot order [Kdim/32][slots][32]: the
-                        // gathered x (mode 0, gather_act_kernel) or h (mode 1)
-    const float* ad;    // their scales (exact fp16 values) [Kdim/32][slots]
-    int T, H, I, E, K;
-    int Kdim;           // reduction length (H for mode 0, I for modes 1/2)
-    int nrb;            // row blocks of the weight matrix
-    int tiles_pad;      // tile bound rounded up to a multiple of MM_XCD x the shape's GROUP (sizes the grid)
-    int8_t* hq;         // mode 0 outputs
-    float* hd;
-    int* hs;
-    float* y;           // mode 1 output
-    int* ctr;           // MM_CTR_INTS work counters, zeroed by gather_act_kernel before the gate/up launch
-};
-
 // Byte offset, inside a 32-byte operand row, of the row's 16-byte half h: the halves
 // are swapped when bit 3 of the row is set (conflict-free MFMA operand reads).
 __device__ __forceinline__ int swz_half(int row, int h) { return 16 * (h ^ ((row >> 3) & 1)); }
@@ -133,18 +114,6 @@ __device__ __forceinline__ int operand_lane_off(int lr, int lg) { return lr * 32
 // 16-31) nibbles of the row's 16 stored bytes; lanes 2j and 2j + 1 read the same
 // nibble row.  nib = the chunk's nibble rows + 16 * (l / 2), dst = its int8 rows + 16 l,
 // sh = 4 - 4 h (the same for rows l / 2 and 32 + l / 2).
-//
-// A weight n - 8 is left in the high nibble of its byte, as the int8 value 16 (n - 8)
-// (n with its top bit flipped is n - 8 in two's complement): a shift and one
-// three-input logic operation per four weights.  Block dots and accumulators come out 16
-// times too large, exactly -- a block dot is at most 16 x 8 x 127 x 32 < 2^24, and the
-// accumulator chain scales by a power of two (its values are multiples of 2^-48, far
-// from denormals) -- and the epilogue multiplies by 1/16.  Against n - 8 itself (five
-// operations per four weights): Q4_0 layers of T = 48 465 -> 454 us, 4096 skewed tokens
-// 3.94 -> 3.92 ms, a decoder layer of T = 300 906 -> 895 us (same box).
-__device__ __forceinline__ int unpack_q4x16(int v, uint32_t sh) {
-    return (int)((((uint32_t)v << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
-}
 __device__ __forceinline__ void unpack_q4_chunk_at(uint32_t nib, uint32_t dst, uint32_t sh) {
     v4i_t w0 = lds_b128_at<0>(nib);
     v4i_t w1 = lds_b128_at<512>(nib);
@@ -154,13 +123,6 @@ __device__ __forceinline__ void unpack_q4_chunk_at(uint32_t nib, uint32_t dst, u
     lds_st128_at<1024>(dst, v4i_t{cv(w1[0]), cv(w1[1]), cv(w1[2]), cv(w1[3])});
 }
 __device__ __forceinline__ uint32_t unpack_q4_shift(int lane) { return 4u - 4u * (uint32_t)((lane & 1) ^ ((lane >> 4) & 1)); }
-
-// The exact int32 dots of one 32-wide GGUF block over a 32x32 tile (K = 32 is one
-// block): v_mfma_i32_32x32x32_i8 with a zero accumulator.
-__device__ __forceinline__ v16i_t block_dot_tile(v4i_t A, v4i_t B) {
-    const v16i_t zero = {};
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, zero, 0, 0, 0);
-}
 
 // Per-block scale products c[row][tok] = d_w[row] * d_x[tok] for a 32x32 tile from one
 // f16 MFMA: A holds d_w in k-slot 0 of lane group 0, B holds d_x in the same slot,
@@ -538,53 +500,10 @@ __global__ __launch_bounds__(SH::THREADS, SH::WG_PER_CU) void moe_mfma_kernel(Mm
                 au[v] *= 0.0625f;
             }
         }
-        if (MODE == 0) {
-            // ag = gate rows, au = matching up rows of slab (MM_SLABS * rb + sl)
-            const int slab = MM_SLABS * rb + sl;
-            float h[16];
-            float amax = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                h[v] = swiglu(ag[v], au[v]);
-                amax = fmaxf(amax, fabsf(h[v]));
-            }
-            amax = fmaxf(amax, __shfl_xor(amax, 32, WAVE));
-            const float d = amax / 127.0f;
-            const float id = d != 0.0f ? 1.0f / d : 0.0f;
-            int qsum = 0;
-            int packed[4];
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                uint32_t p = 0;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int q = (int)__builtin_roundf(h[4 * g + i] * id);
-                    qsum += q;
-                    p |= ((uint32_t)(q & 0xff)) << (8 * i);
-                }
-                packed[g] = (int)p;
-            }
-            qsum += __shfl_xor(qsum, 32, WAVE);
-            // h block-major: block (slab) plane, slot row of 32 bytes
-            const size_t hi = (size_t)slab * (size_t)(a.T * a.K + a.T) + (size_t)slot_s[j];
-            int8_t* dst = a.hq + hi * QK;
-#pragma unroll
-            for (int g = 0; g < 4; g++) *reinterpret_cast<int*>(dst + 8 * g + 4 * lg) = packed[g];
-            if (lg == 0) {
-                a.hd[hi] = h2f(f2h(d));
-                a.hs[hi] = qsum;
-            }
-        } else {
-            const int rbase = row0 + sl * 64;
-            float* yr = a.y + (size_t)slot_s[j] * a.H;
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int r = 8 * g + 4 * lg;
-                *reinterpret_cast<float4*>(yr + rbase + r) = make_float4(ag[4 * g], ag[4 * g + 1], ag[4 * g + 2], ag[4 * g + 3]);
-                *reinterpret_cast<float4*>(yr + rbase + 32 + r) =
-                    make_float4(au[4 * g], au[4 * g + 1], au[4 * g + 2], au[4 * g + 3]);
-            }
-        }
+        if (MODE == 0)
+            mm_store_h(a, ag, au, MM_SLABS * rb + sl, slot_s[j], lg);
+        else
+            mm_store_y(a, ag, au, row0 + sl * 64, slot_s[j], lg);
     };
     if (!active) return;
     const int j0 = nq * 32 * TT + lr;  // pair index within the tile
@@ -710,6 +629,8 @@ static hipError_t launch_mode(int wtype, MmArgs a, int n_tiles_bound, int rows, 
 
 template <int MODE>
 static hipError_t launch_shape(int wtype, int shape, MmArgs a, int n_tiles_bound, int rows, hipStream_t s) {
+    if (shape == MM_SHAPE_FEW)
+        return MODE == 0 ? launch_up_few(wtype, n_tiles_bound, a, s) : launch_down_few(wtype, n_tiles_bound, a, s);
     if (shape == MM_SHAPE_TALL) return launch_mode<MODE, ShapeTall>(wtype, a, n_tiles_bound, rows, s);
     return launch_mode<MODE, ShapeWide>(wtype, a, n_tiles_bound, rows, s);
 }
@@ -723,16 +644,20 @@ bool mfma_path_ok(int wtype, int H, int I) {
     return (wtype == HY_TYPE_Q8_0 || wtype == HY_TYPE_Q4_0) && shape_fits<ShapeWide>(H, I);
 }
 
-// The tall shape (64-pair tiles, 256-row blocks) wins while experts see about 64
-// pairs each (a 128-pair tile would leave half its waves idle); beyond ~96 the wide
+// The stream of hy_mfma_few.hip wins while most experts fit one of its 32-pair tiles (a
+// second tile streams the weights again): H 4096, I 3072, E 64, K 8, few against tall:
+// T = 192 (24 pairs per expert) Q4_0 385 / 485 us, Q8_0 527 / 572; T = 256 519 / 524 and
+// 630 / 599.  The tall shape (64-pair tiles, 256-row blocks) wins while experts see about
+// 64 pairs each (a 128-pair tile would leave half its waves idle); beyond ~96 the wide
 // shape's reuse of every weight byte over 128 pairs wins.
 int mfma_shape(int T, int K, int E, int H, int I) {
+    if ((int64_t)T * K <= (int64_t)24 * E) return MM_SHAPE_FEW;
     const bool tall = shape_fits<ShapeTall>(H, I) && (int64_t)T * K < (int64_t)96 * E;
     return tall ? MM_SHAPE_TALL : MM_SHAPE_WIDE;
 }
 
 int mfma_shape_tokens(int shape) {
-    return shape == MM_SHAPE_TALL ? ShapeTall::TOK : ShapeWide::TOK;
+    return shape == MM_SHAPE_FEW ? FEW_TOK : shape == MM_SHAPE_TALL ? ShapeTall::TOK : ShapeWide::TOK;
 }
 
 hipError_t launch_gather_act(const ActQ& X, const Routing& R, int T, int K, int H, int8_t* gq, float* gd,
