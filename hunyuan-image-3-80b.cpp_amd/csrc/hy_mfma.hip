@@ -644,15 +644,19 @@ bool mfma_path_ok(int wtype, int H, int I) {
     return (wtype == HY_TYPE_Q8_0 || wtype == HY_TYPE_Q4_0) && shape_fits<ShapeWide>(H, I);
 }
 
-// The stream of hy_mfma_few.hip wins while most experts fit one of its 32-pair tiles (a
-// second tile streams the weights again): H 4096, I 3072, E 64, K 8, few against tall:
-// T = 192 (24 pairs per expert) Q4_0 385 / 485 us, Q8_0 527 / 572; T = 256 519 / 524 and
-// 630 / 599.  The tall shape (64-pair tiles, 256-row blocks) wins while experts see about
-// 64 pairs each (a 128-pair tile would leave half its waves idle); beyond ~96 the wide
-// shape's reuse of every weight byte over 128 pairs wins.
-int mfma_shape(int T, int K, int E, int H, int I) {
-    if ((int64_t)T * K <= (int64_t)24 * E) return MM_SHAPE_FEW;
-    const bool tall = shape_fits<ShapeTall>(H, I) && (int64_t)T * K < (int64_t)96 * E;
+// The stream of hy_mfma_few.hip wins while most experts fit one of its 32-pair tiles, as a
+// second tile streams the weights again: H 4096, I 3072, E 64, K 8, few against tall: T = 208
+// (26 pairs per expert) Q4_0 381 / 483 us, Q8_0 533 / 578; T = 240 444 / 494 and 640 / 592.
+// Where the gate/up weights fit the Infinity Cache a second tile finds them there: H 2048,
+// I 1536, E 16, K 4: T = 200 (50 pairs) Q4_0 90 / 115, Q8_0 95 / 109; T = 300 102 / 129
+// and 104 / 123.  The tall shape (64-pair tiles, 256-row blocks) wins while experts see
+// about 64 pairs each (a 128-pair tile would leave half its waves idle); beyond ~96 the
+// wide shape's reuse of every weight byte over 128 pairs wins.
+int mfma_shape(int wtype, int T, int K, int E, int H, int I) {
+    const int64_t pairs = (int64_t)T * K;
+    const bool cached = (size_t)(E + 1) * 2 * I * (H / QK) * block_bytes(wtype) <= INFINITY_CACHE;
+    if (pairs <= (int64_t)(cached ? 64 : 26) * E) return MM_SHAPE_FEW;
+    const bool tall = shape_fits<ShapeTall>(H, I) && pairs < (int64_t)96 * E;
     return tall ? MM_SHAPE_TALL : MM_SHAPE_WIDE;
 }
 

@@ -50,6 +50,7 @@ __device__ __forceinline__ v16i_t block_dot_tile(v4i_t A, v4i_t B) {
 
 // the products of tiles of up to FEW_TOK pairs (hy_mfma_few.hip)
 constexpr int FEW_TOK = 32;
+constexpr size_t INFINITY_CACHE = (size_t)256 << 20;
 hipError_t launch_up_few(int wtype, int n_tiles_bound, const MmArgs& a, hipStream_t s);
 hipError_t launch_down_few(int wtype, int n_tiles_bound, const MmArgs& a, hipStream_t s);
 

@@ -21,8 +21,7 @@
 
 namespace hy {
 
-constexpr int FEW_D = 4;                           // blocks in registers, one of them in use
-constexpr size_t FEW_NT_BYTES = (size_t)256 << 20;  // the Infinity Cache
+constexpr int FEW_D = 4;  // blocks in registers, one of them in use
 
 template <int WT, int MODE, bool NT>
 __global__ __launch_bounds__(256, 3) void moe_few_kernel(MmArgs a) {
@@ -119,7 +118,7 @@ template <int WT, int MODE>
 static hipError_t few_launch(MmArgs a, int n_tiles_bound, int rows, hipStream_t s) {
     a.nrb = (rows / 64 + 3) / 4;
     const dim3 grid((unsigned)(n_tiles_bound * a.nrb));
-    if (a.W.qs_stride * (size_t)a.W.n_mats > FEW_NT_BYTES)
+    if (a.W.qs_stride * (size_t)a.W.n_mats > INFINITY_CACHE)
         hipLaunchKernelGGL((moe_few_kernel<WT, MODE, true>), grid, dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((moe_few_kernel<WT, MODE, false>), grid, dim3(256), 0, s, a);

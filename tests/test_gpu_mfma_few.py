@@ -15,10 +15,10 @@ pytestmark = pytest.mark.gpu
 def test_few(gpu, wtype, H, I, shared):
     E, K = 3, 2
     layer = O.synth_layer(H, I, E, K, wtype, seed=H + I, std=0.05, shared=shared)
-    m = gpu.Moe(H, I, E, K, wtype, max_tokens=64, has_shared=shared)
+    m = gpu.Moe(H, I, E, K, wtype, max_tokens=128, has_shared=shared)
     m.set_path(gpu.PATH_MFMA)
     m.upload(0, layer)
-    for T in (1, 2, 16, 17, 31, 32, 33, 36, 37):  # 24 pairs per expert end at T = 36
+    for T in (1, 2, 16, 17, 31, 32, 33, 96, 97):  # 64 pairs per expert end at T = 96
         x = O.synth(70 + T, 0, O.T_X, 0, (T, H), 1.0)
         got, ref = m.run(0, x), O.moe_forward_q(layer, x)
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), f"T={T}"
