@@ -137,8 +137,49 @@ __global__ __launch_bounds__(256) void rms_norm_w_kernel(const float* __restrict
     for (int h = lane; h < H; h += WAVE) out[(size_t)row * H + h] = xr[h] * rms * w[h];
 }
 
+// The same for H a multiple of 256 up to 4096, one work group per row: every wave loads the
+// whole row into registers at once and forms the whole sum (the same order, so the same
+// bits), then writes every fourth chunk.  Bound: latency; one wave per row with one load in
+// flight took 30 us at T = 300, H = 4096 (this: 6).
+constexpr int RMSW_MAX_CHUNKS = 16;
+__global__ __launch_bounds__(256) void rms_norm_w_reg_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                             int H, float eps, float* __restrict__ out) {
+    const int row = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const int nc = H / (4 * WAVE);
+    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * H) + lane;
+    float4 v[RMSW_MAX_CHUNKS];
+#pragma unroll
+    for (int i = 0; i < RMSW_MAX_CHUNKS; i++)
+        if (i < nc) v[i] = xr[WAVE * i];
+    float a = 0.0f;
+#pragma unroll
+    for (int i = 0; i < RMSW_MAX_CHUNKS; i++)
+        if (i < nc) {
+            a = fmaf(v[i].x, v[i].x, a);
+            a = fmaf(v[i].y, v[i].y, a);
+            a = fmaf(v[i].z, v[i].z, a);
+            a = fmaf(v[i].w, v[i].w, a);
+        }
+    const float ss = __shfl(tree_sum64(a), 0, WAVE);
+    __syncthreads();  // out may be x: no wave writes before all have read
+    const float rms = 1.0f / sqrtf(ss / (float)H + eps);
+    const float4* wr = reinterpret_cast<const float4*>(w) + lane;
+    float4* o = reinterpret_cast<float4*>(out + (size_t)row * H) + lane;
+#pragma unroll
+    for (int i = 0; i < RMSW_MAX_CHUNKS; i++)
+        if (i < nc && i % 4 == wave) {
+            const float4 ww = wr[WAVE * i];
+            o[WAVE * i] = make_float4(v[i].x * rms * ww.x, v[i].y * rms * ww.y, v[i].z * rms * ww.z, v[i].w * rms * ww.w);
+        }
+}
+
 hipError_t launch_rms_norm_w(const float* x, const float* w, int T, int H, float eps, float* out, hipStream_t s) {
-    hipLaunchKernelGGL(rms_norm_w_kernel, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, out);
+    // 16-byte rows and pointers: whatever a caller passes is aligned to its floats only
+    const bool vec = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
+    if (vec && H % (4 * WAVE) == 0 && H <= 4 * WAVE * RMSW_MAX_CHUNKS)
+        hipLaunchKernelGGL(rms_norm_w_reg_kernel, dim3(T), dim3(256), 0, s, x, w, H, eps, out);
+    else
+        hipLaunchKernelGGL(rms_norm_w_kernel, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, out);
     return hipGetLastError();
 }
 

@@ -83,8 +83,8 @@ __device__ __forceinline__ void topk_groups_wave(float v_in, int E, int K, int n
 
 // Router logits.  Work item of one wave = (TPW tokens) x (EPW experts); a block's
 // four waves take consecutive items, experts varying fastest so they share the
-// token rows in L1.  Decode batches (T <= 16) use <1,1> (one dot per wave), T <= 32
-// <8,1>, up to 2047 tokens <4,8> (each Wr float4 feeds 4 tokens, 32 accumulators per
+// token rows in L1.  Decode batches (T <= 16) use <1,1> (one dot per wave), T <= 128
+// <2,4>, up to 2047 tokens <4,8> (each Wr float4 feeds 4 tokens, 32 accumulators per
 // lane), larger batches <8,8>: each loaded float4 feeds 8 dots, 64 accumulators per lane
 // (1.05 GB of L2 reads at T=4096 against 1.57 GB for <4,8>: 61 vs 78 us; at T=512 its
 // 512 waves are too few, 27 vs 23 us).  The
@@ -257,8 +257,10 @@ hipError_t launch_router_q(const float* x, const float* wr, int T, int H, int E,
         // decode batches: one (token, expert) item per wave, T x E waves; a wave that
         // covers several tokens serialises their dot products (9.3 vs 4.5 us at T=8)
         hipLaunchKernelGGL((router_logits_kernel<1, 1>), grid_for(1, 1), blk, 0, s, x, wr, T, H, E, logits);
-    } else if (T <= 32) {
-        hipLaunchKernelGGL((router_logits_kernel<8, 1>), grid_for(8, 1), blk, 0, s, x, wr, T, H, E, logits);
+    } else if (T <= 128) {
+        // a wave's chunks in flight, not its loads, set the time of so few waves: twice the
+        // depth of <4,8> (T = 48, H = 4096, E = 64: 16.6 -> 7.4 us)
+        hipLaunchKernelGGL((router_logits_kernel<2, 4>), grid_for(2, 4), blk, 0, s, x, wr, T, H, E, logits);
     } else {
         // full chunks: H a multiple of D x 256 elements
         auto full = [&](int d) { return H % (4 * WAVE * d) == 0; };
@@ -477,7 +479,8 @@ hipError_t launch_quant_q8_0(const float* x, size_t n, int8_t* q, float* d, int*
 // list is therefore the reference's dispatch_mask slot c.  Also builds the per-token
 // combine lists (pairs in ascending expert order, the einsum_combine summation
 // order of :387-397) and a list of tiles of at most NT pairs.
-// Three launches, no atomics outside LDS:
+// Up to 1024 pairs: one launch (dispatch_small_kernel).  More: three launches, no atomics
+// outside LDS:
 //  1. dispatch_rank_kernel, one work group per (block of 1024 tokens, rank k): an LDS
 //     bitmap of the block's tokens per expert gives each pair its rank among the
 //     block's pairs of that expert and rank, and the block's count per expert;
@@ -543,6 +546,46 @@ __global__ __launch_bounds__(DSP_BLOCK) void dispatch_rank_kernel(const int* __r
         rank[(size_t)t * K + k] = wpre[e][tid / 32] + __popc(mask[e][tid / 32] & ((1u << (tid % 32)) - 1u));
 }
 
+// expert offsets, tiles and totals from the pairs per expert (one wave; cnt_s in LDS);
+// returns the lane's expert's offset
+__device__ __forceinline__ int dispatch_lists(const int* cnt_s, int lane, int T, int E, int NT, int has_shared, int cap,
+                                              const DispatchOut& o) {
+    // c pairs of the expert, the first min(c, cap) of them computed (capacity slots,
+    // src/hunyuan_moe_full.cpp:296-304: a pair at slot >= capacity is dropped)
+    const int c = lane < E ? cnt_s[lane] : 0;
+    const int kc = c < cap ? c : cap;
+    const int nt = (kc + NT - 1) / NT;
+    const int off = wave_excl_scan(c, lane), toff = wave_excl_scan(nt, lane);
+    const int total = __shfl(off + c, WAVE - 1, WAVE), routed = __shfl(toff + nt, WAVE - 1, WAVE);
+    const int distinct = __popcll(__ballot(c > 0));
+    const int ns = has_shared ? (T + NT - 1) / NT : 0;
+    if (lane < E) {
+        o.cnt[lane] = c;
+        o.off[lane] = off;
+        o.meta[META_TILE_OFF + lane] = toff;
+        for (int j = 0; j < nt; j++) {
+            o.tile_e[toff + j] = lane;
+            o.tile_start[toff + j] = j * NT;
+            o.tile_n[toff + j] = min(NT, kc - j * NT);
+        }
+    }
+    if (lane == 0) {
+        o.off[E] = total;
+        o.meta[0] = routed;
+        o.meta[1] = routed + ns;
+        o.meta[2] = distinct;
+        o.meta[3] = T;
+        o.meta[META_TILE_OFF + E] = routed;
+        o.meta[META_TILE_OFF + E + 1] = routed + ns;
+    }
+    for (int j = lane; j < ns; j += WAVE) {
+        o.tile_e[routed + j] = E;
+        o.tile_start[routed + j] = j * NT;
+        o.tile_n[routed + j] = min(NT, T - j * NT);
+    }
+    return off;
+}
+
 // blk_cnt [K][nblk][E] (k-major: the priority order) -> exclusive bases in place
 __global__ __launch_bounds__(256) void dispatch_scan_kernel(int T, int K, int E, int NT, int has_shared, int nblk,
                                                             int cap, int* __restrict__ blk_cnt, DispatchOut o) {
@@ -566,41 +609,7 @@ __global__ __launch_bounds__(256) void dispatch_scan_kernel(int T, int K, int E,
         cnt_s[tid] = run;
     }
     __syncthreads();
-    if (tid < WAVE) {
-        // c pairs of the expert, the first min(c, cap) of them computed (capacity slots,
-        // src/hunyuan_moe_full.cpp:296-304: a pair at slot >= capacity is dropped)
-        const int c = lane < E ? cnt_s[lane] : 0;
-        const int kc = c < cap ? c : cap;
-        const int nt = (kc + NT - 1) / NT;
-        const int off = wave_excl_scan(c, lane), toff = wave_excl_scan(nt, lane);
-        const int total = __shfl(off + c, WAVE - 1, WAVE), routed = __shfl(toff + nt, WAVE - 1, WAVE);
-        const int distinct = __popcll(__ballot(c > 0));
-        const int ns = has_shared ? (T + NT - 1) / NT : 0;
-        if (lane < E) {
-            o.cnt[lane] = c;
-            o.off[lane] = off;
-            o.meta[META_TILE_OFF + lane] = toff;
-            for (int j = 0; j < nt; j++) {
-                o.tile_e[toff + j] = lane;
-                o.tile_start[toff + j] = j * NT;
-                o.tile_n[toff + j] = min(NT, kc - j * NT);
-            }
-        }
-        if (lane == 0) {
-            o.off[E] = total;
-            o.meta[0] = routed;
-            o.meta[1] = routed + ns;
-            o.meta[2] = distinct;
-            o.meta[3] = T;
-            o.meta[META_TILE_OFF + E] = routed;
-            o.meta[META_TILE_OFF + E + 1] = routed + ns;
-        }
-        for (int j = lane; j < ns; j += WAVE) {
-            o.tile_e[routed + j] = E;
-            o.tile_start[routed + j] = j * NT;
-            o.tile_n[routed + j] = min(NT, T - j * NT);
-        }
-    }
+    if (tid < WAVE) dispatch_lists(cnt_s, lane, T, E, NT, has_shared, cap, o);
 }
 
 __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int* __restrict__ topi,
@@ -618,6 +627,55 @@ __global__ __launch_bounds__(256) void dispatch_scatter_kernel(const int* __rest
     o.srt_tok[pos] = t;
     // combine list slot: the token's experts are distinct, so the pair's place in
     // ascending expert order is the count of the token's smaller experts
+    int r = 0;
+    for (int j = 0; j < K; j++) r += topi[(size_t)t * K + j] < e;
+    o.comb_pos[(size_t)t * K + r] = pos;
+    o.comb_w[(size_t)t * K + r] = slot < cap ? topw[p] : 0.0f;  // a dropped pair adds nothing
+}
+
+// The whole dispatch of at most DSP_BLOCK pairs in one launch: thread i owns flat slot i =
+// k T + t, so one bitmap of the slots per expert gives the pair's place in its expert's
+// list.  Three launches of such a batch are 15 us of which 9 are boundaries; this is one
+// of 6.
+__global__ __launch_bounds__(DSP_BLOCK) void dispatch_small_kernel(const int* __restrict__ topi,
+                                                                  const float* __restrict__ topw, int T, int K, int E,
+                                                                  int NT, int has_shared, int cap, DispatchOut o) {
+    __shared__ uint32_t mask[MAX_E][DSP_BLOCK / 32];
+    __shared__ int wpre[MAX_E][DSP_BLOCK / 32];
+    __shared__ int cnt_s[MAX_E], off_s[MAX_E];
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    for (int i = tid; i < MAX_E * (DSP_BLOCK / 32); i += DSP_BLOCK) (&mask[0][0])[i] = 0u;
+    __syncthreads();
+    const int k = tid / T, t = tid - k * T, p = t * K + k;
+    int e = k < K ? topi[p] : -1;
+    if (e >= E) e = -1;  // an out-of-range id is dropped (never produced by the router)
+    if (e >= 0) atomicOr(&mask[e][tid / 32], 1u << (tid % 32));
+    __syncthreads();
+    for (int i = tid; i < MAX_E * (DSP_BLOCK / 32); i += DSP_BLOCK) {
+        const int ee = i / 32, w = i % 32;
+        const int c = __popc(mask[ee][w]);
+        int incl = c;
+#pragma unroll
+        for (int d = 1; d < 32; d <<= 1) {
+            const int u = __shfl_up(incl, d, 32);
+            if (w >= d) incl += u;
+        }
+        wpre[ee][w] = incl - c;
+        if (w == 31) cnt_s[ee] = incl;
+    }
+    __syncthreads();
+    if (tid < WAVE) {
+        const int off = dispatch_lists(cnt_s, lane, T, E, NT, has_shared, cap, o);
+        if (lane < MAX_E) off_s[lane] = off;
+    }
+    __syncthreads();
+    if (e < 0) return;
+    const int slot = wpre[e][tid / 32] + __popc(mask[e][tid / 32] & ((1u << (tid % 32)) - 1u));
+    const int pos = off_s[e] + slot;
+    o.pair_pos[p] = pos;
+    o.srt_tok[pos] = t;
+    // the token's experts are distinct: the pair's place in ascending expert order is the
+    // count of its smaller experts
     int r = 0;
     for (int j = 0; j < K; j++) r += topi[(size_t)t * K + j] < e;
     o.comb_pos[(size_t)t * K + r] = pos;
@@ -839,6 +897,11 @@ hipError_t launch_dispatch(const int* topi, const float* topw, int T, int K, int
                            int* cnt, int* off, int* srt_tok, int* pair_pos, int* comb_pos, float* comb_w,
                            int* tile_e, int* tile_start, int* tile_n, int* meta, int* scratch, hipStream_t s, int cap) {
     DispatchOut o{cnt, off, srt_tok, pair_pos, comb_pos, comb_w, tile_e, tile_start, tile_n, meta};
+    if ((int64_t)T * K <= DSP_BLOCK) {
+        hipLaunchKernelGGL(dispatch_small_kernel, dim3(1), dim3(DSP_BLOCK), 0, s, topi, topw, T, K, E, NT, has_shared,
+                           cap, o);
+        return hipGetLastError();
+    }
     const int nblk = (T + DSP_BLOCK - 1) / DSP_BLOCK;
     hipLaunchKernelGGL(dispatch_rank_kernel, dim3(nblk, K), dim3(DSP_BLOCK), 0, s, topi, T, K, E, scratch, pair_pos);
     hipError_t e = hipGetLastError();
@@ -962,13 +1025,17 @@ __global__ __launch_bounds__(256) void rms_norm_quant_kernel(const float* __rest
 // The same RMSNorm + Q8_0 with the row read once: for H a multiple of 256 up to 4096 a
 // lane keeps its 4 H/256 elements (4 lane + 256 i .. +3, the sum-of-squares order)
 // in registers, and the 8 lanes holding one 32-wide block reduce its amax and sum.
-// Same values bit for bit.
+// Same values bit for bit.  WPR = 4: a work group per row, whose waves all form the sum and
+// then quantize every fourth chunk each, for batches that leave the chip's waves idle
+// (T = 300, H = 4096: 9 us where one wave per row takes 16).
 constexpr int RMSQ_MAX_CHUNKS = 16;
+template <int WPR>
 __global__ __launch_bounds__(256) void rms_norm_quant_reg_kernel(const float* __restrict__ x,
                                                                  const float* __restrict__ w, int T, int H, float eps,
                                                                  float* __restrict__ xn, int8_t* __restrict__ q,
                                                                  float* __restrict__ d, int* __restrict__ qsum) {
-    const int row = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const int row = WPR == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
     if (row >= T) return;  // whole waves: the shuffles below stay within live waves
     const int nc = H / (4 * WAVE);
     const float* xr = x + (size_t)row * H;
@@ -986,11 +1053,12 @@ __global__ __launch_bounds__(256) void rms_norm_quant_reg_kernel(const float* __
             a = fmaf(v[i].w, v[i].w, a);
         }
     const float ss = __shfl(tree_sum64(a), 0, WAVE);
+    if (WPR == 4) __syncthreads();  // xn may be x: no wave writes before all have read
     const float rms = 1.0f / sqrtf(ss / (float)H + eps);
     const int nb = H / QK;
 #pragma unroll
     for (int i = 0; i < RMSQ_MAX_CHUNKS; i++) {
-        if (i >= nc) continue;  // (uniform; keeps the loop unrolled and v[] in registers)
+        if (i >= nc || (WPR == 4 && i % 4 != wave)) continue;  // (uniform; keeps the loop unrolled and v[] in registers)
         const int h = 4 * lane + 4 * WAVE * i;
         float xs[4] = {v[i].x * rms, v[i].y * rms, v[i].z * rms, v[i].w * rms};
         if (w) {
@@ -1030,8 +1098,11 @@ __global__ __launch_bounds__(256) void rms_norm_quant_reg_kernel(const float* __
 hipError_t launch_rms_norm_quant(const float* x, const float* w, int T, int H, float eps, float* xn, int8_t* q,
                                  float* d, int* qsum, hipStream_t s) {
     if (H % (4 * WAVE) == 0 && H <= 4 * WAVE * RMSQ_MAX_CHUNKS)
-        hipLaunchKernelGGL(rms_norm_quant_reg_kernel, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, xn, q, d,
-                           qsum);
+        if (T < 2048)
+            hipLaunchKernelGGL(rms_norm_quant_reg_kernel<4>, dim3(T), dim3(256), 0, s, x, w, T, H, eps, xn, q, d, qsum);
+        else
+            hipLaunchKernelGGL(rms_norm_quant_reg_kernel<1>, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, xn, q,
+                               d, qsum);
     else
         hipLaunchKernelGGL(rms_norm_quant_kernel, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, xn, q, d,
                            qsum);
