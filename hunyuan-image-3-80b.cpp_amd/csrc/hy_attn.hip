@@ -111,8 +111,8 @@ __global__ __launch_bounds__(WAVE * WM * WN) void gemm_nt_f32_kernel(const float
 // (the same for all waves: L1 hits) feeds GV_RPW rows.  Loads are unconditional from
 // clamped addresses and software-pipelined GV_D chunks deep; a chunk past K is masked
 // by a select.  The 64 lane partials of every output fold level by level at the end.
-constexpr int GV_RPW = 2;  // two rows per wave: 4 KB in flight per wave at depth 4 (swept 1..8)
-template <int MB, int GV_D>
+// Two rows per wave and 4 KB in flight at depth 4 (swept 1..8) up to 8 rows of A.
+template <int MB, int GV_D, int GV_RPW>
 __global__ __launch_bounds__(256) void gemv_nt_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                          const float* __restrict__ R, float* __restrict__ C, int M,
                                                          int N, int K) {
@@ -195,21 +195,37 @@ bool gemm_nt_f32_uses_ws(int M, int N, int K) {
 hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                               hipStream_t s, float* ws) {
     if (M <= 16) {
-        const dim3 grid((unsigned)((N + 4 * GV_RPW - 1) / (4 * GV_RPW)));
-        // rows 8.. go through a second pass over W (M <= 16 keeps it at two)
-        for (int m0 = 0; m0 < M; m0 += 8) {
-            const int mb = min(M - m0, 8);
-            const float* a = A + (size_t)m0 * K;
-            const float* r = R ? R + (size_t)m0 * N : nullptr;
-            float* c = C + (size_t)m0 * N;
-            if (mb == 1)
-                hipLaunchKernelGGL((gemv_nt_f32_kernel<1, 4>), grid, dim3(256), 0, s, a, W, r, c, mb, N, K);
-            else if (mb == 2)
-                hipLaunchKernelGGL((gemv_nt_f32_kernel<2, 4>), grid, dim3(256), 0, s, a, W, r, c, mb, N, K);
-            else if (mb <= 4)
-                hipLaunchKernelGGL((gemv_nt_f32_kernel<4, 4>), grid, dim3(256), 0, s, a, W, r, c, mb, N, K);
+        using std::integral_constant;
+        auto gemv = [&](auto mb, auto depth, auto rpw, int m0, int m) {
+            constexpr int MB = decltype(mb)::value, D = decltype(depth)::value, RPW = decltype(rpw)::value;
+            hipLaunchKernelGGL((gemv_nt_f32_kernel<MB, D, RPW>), dim3((unsigned)((N + 4 * RPW - 1) / (4 * RPW))),
+                               dim3(256), 0, s, A + (size_t)m0 * K, W, R ? R + (size_t)m0 * N : nullptr,
+                               C + (size_t)m0 * N, m, N, K);
+        };
+        const integral_constant<int, 2> two{};
+        const integral_constant<int, 3> three{};
+        const integral_constant<int, 4> four{};
+        // 9 to 16 rows of A in one pass over W, four W rows per wave (each A float4 read
+        // feeds them all), where N leaves a wave for every SIMD: 4096 -> 6144 and back, whole
+        // attention, T = 9 84 -> 67 us, T = 16 102 -> 83.  Fewer rows of W run two passes of
+        // eight on twice the waves (1024 -> 1536 and back: T = 16 36 us, one pass 39).
+        if (M > 8 && N >= 4096) {
+            if (M <= 12)
+                gemv(integral_constant<int, 12>{}, two, four, 0, M);
             else
-                hipLaunchKernelGGL((gemv_nt_f32_kernel<8, 3>), grid, dim3(256), 0, s, a, W, r, c, mb, N, K);
+                gemv(integral_constant<int, 16>{}, two, four, 0, M);
+            return hipGetLastError();
+        }
+        for (int m0 = 0; m0 < M; m0 += 8) {
+            const int m = min(M - m0, 8);
+            if (m == 1)
+                gemv(integral_constant<int, 1>{}, four, two, m0, m);
+            else if (m == 2)
+                gemv(two, four, two, m0, m);
+            else if (m <= 4)
+                gemv(four, four, two, m0, m);
+            else
+                gemv(integral_constant<int, 8>{}, three, two, m0, m);
         }
         return hipGetLastError();
     }

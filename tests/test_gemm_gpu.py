@@ -90,3 +90,19 @@ def test_errors_have_no_mean(gpu, M, N, K):
     w = rng.standard_normal((N, K)).astype(np.float32)
     e = gpu.lm_head_f32(x, w) - x.astype(np.float64) @ w.astype(np.float64).T
     assert abs(e.mean()) <= 0.025 * np.sqrt((e * e).mean())
+
+
+# nine to sixteen rows in one pass (N of 4096 and more, not a multiple of a wave's four rows)
+# and in two; K past and below the lanes' chunks
+@pytest.mark.parametrize("M", [9, 12, 13, 16])
+@pytest.mark.parametrize("N,K", [(4096, 272), (5003, 1040), (4095, 1024)])
+def test_nine_to_sixteen_rows(gpu, M, N, K):
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    r = rng.standard_normal((M, N)).astype(np.float32)
+    got = gpu.lm_head_f32(x, w)
+    check(got, x, w)
+    check(gpu.lm_head_f32(x, w, r), x, w, r)
+    # a row's bits do not depend on how many rows share the pass
+    assert np.array_equal(got[:8].view(np.uint32), gpu.lm_head_f32(x[:8], w).view(np.uint32))
