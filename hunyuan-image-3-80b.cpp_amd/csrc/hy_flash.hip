@@ -21,6 +21,10 @@
 //
 // Values without a split (infinities, NaNs, values that round up to infinity in bf16)
 // leave a non-finite sum: such a wave computes its keys again on the fp32 matrix cores.
+// So do the waves that met a q, k or v too small for an exact split.  The probabilities
+// are taken 2^40 times too large, which keeps the split of each of them exact (they are 0 or
+// at least 2^-126, the split needs 2^-110); the sum of the values and the sum of the
+// probabilities carry the factor alike.
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
 #include "hy_lds.hpp"
@@ -29,6 +33,7 @@
 namespace hy {
 
 constexpr int FS_TURN = 4;  // key blocks of one accumulator sign
+constexpr float FS_PSCALE = 0x1p40f;  // of the probabilities
 
 template <int HD>
 struct FsLds {
@@ -49,6 +54,7 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
     constexpr int ND = HD / 32;  // 32-dim tiles of the output
     constexpr int NK = HD / 64;  // float4s of K, and dims of V, per thread and block
     __shared__ __attribute__((aligned(1024))) uint8_t lds[L::BYTES];
+    __shared__ int lost_s;  // an inexact split of K or V
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int lr = lane % 32, h = lane / 32;
@@ -99,8 +105,10 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
             for (int i = 0; i < NK; i++) vx[i][j] = row[32 * i];
         }
     };
+    uint32_t lost = 0;
+    if (tid == 0) lost_s = 0;
     auto put = [&](uint8_t* dst, int piece, v4f_t x) {
-        const Split2 s = split2(x[0], x[1]), t = split2(x[2], x[3]);
+        const Split2 s = split2(x[0], x[1], lost), t = split2(x[2], x[3], lost);
 #pragma unroll
         for (int q = 0; q < 3; q++) *reinterpret_cast<uint2*>(dst + q * piece) = make_uint2(s.p[q], t.p[q]);
     };
@@ -126,12 +134,13 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
     const float qscale = a.scale * 1.4426950408889634f;
     const float* const qp = a.q + ((size_t)qrow * a.nh + head) * HD;
     v4i_t qf[NC][3];
+    uint32_t q_lost = 0;
 #pragma unroll
     for (int c = 0; c < NC; c++)
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             const v4f_t x = *reinterpret_cast<const v4f_t*>(qp + 16 * c + 8 * u + 4 * h) * qscale;
-            const Split2 s = split2(x[0], x[1]), t = split2(x[2], x[3]);
+            const Split2 s = split2(x[0], x[1], q_lost), t = split2(x[2], x[3], q_lost);
 #pragma unroll
             for (int q = 0; q < 3; q++) {
                 qf[c][q][2 * u] = (int)s.p[q];
@@ -155,8 +164,8 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
             }
         }
     };
-    // online softmax over this lane pair's 32 keys; s becomes the probabilities
-    auto softmax = [&](v16f_t& s) {
+    // online softmax over this lane pair's 32 keys; s becomes the probabilities times pscale
+    auto softmax = [&](v16f_t& s, float pscale) {
         float mloc = s[0];
 #pragma unroll
         for (int v = 1; v < 16; v++) mloc = fmaxf(mloc, s[v]);
@@ -167,7 +176,7 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
         float psum = 0.0f;
 #pragma unroll
         for (int v = 0; v < 16; v++) {
-            s[v] = __builtin_amdgcn_exp2f(s[v] - m_new);
+            s[v] = __builtin_amdgcn_exp2f(s[v] - m_new) * pscale;
             psum += s[v];
         }
         psum += __shfl_xor(psum, 32, WAVE);
@@ -201,12 +210,13 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         }
         mask(kb, s);
-        const float alpha = softmax(s);
+        const float alpha = softmax(s, FS_PSCALE);
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const Split2 t = split2(s[8 * c + 2 * j], s[8 * c + 2 * j + 1]);
+                uint32_t none = 0;  // exact
+                const Split2 t = split2(s[8 * c + 2 * j], s[8 * c + 2 * j + 1], none);
 #pragma unroll
                 for (int q = 0; q < 3; q++) pf[c][q][j] = (int)t.p[q];
             }
@@ -254,26 +264,34 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
         load_k(kb + 2);
         if (half == 0 && kb < my_kb1) values(kb, alpha);
     }
+    if (lost_bits(lost)) lost_s = 1;
+    __syncthreads();
     if (kb0 >= my_kb1) return;
     if (half == 1 && my_kb1 == kb1) values(kb1 - 1, alpha);
     if (turn_sign<FS_TURN>(my_kb1 - 1 - kb0) < 0.0f) {
 #pragma unroll
         for (int d = 0; d < ND; d++) o[d] = -o[d];
     }
-    bool bad = non_finite(l_run);
+    bool bad = non_finite(l_run) || lost_bits(q_lost) || lost_s;
 #pragma unroll
     for (int d = 0; d < ND; d++)
 #pragma unroll
         for (int v = 0; v < 16; v++) bad |= non_finite(o[d][v]);
+    float unscale = 1.0f / FS_PSCALE;
     if (__any(bad)) {  // again on the fp32 matrix cores, K and V straight from memory
+        unscale = 1.0f;
         reset();
         for (int kb = kb0; kb < my_kb1; kb++) {
-            const float* const k = kg + (size_t)min(kb * 32 + lr, a.kv_len - 1) * HD + h;
+            const float* const k = kg + (size_t)min(kb * 32 + lr, a.kv_len - 1) * HD + 4 * h;
             v16f_t s = v16f_t{};
-            for (int d = 0; d < HD; d += 2)
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[d], qp[d + h] * qscale, s, 0, 0, 0);
+            for (int d = 0; d < HD; d += 8) {
+                const v4f_t kx = *reinterpret_cast<const v4f_t*>(k + d);
+                const v4f_t qx = *reinterpret_cast<const v4f_t*>(qp + d + 4 * h) * qscale;
+#pragma unroll
+                for (int j = 0; j < 4; j++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[j], qx[j], s, 0, 0, 0);
+            }
             mask(kb, s);
-            rescale(softmax(s));
+            rescale(softmax(s, 1.0f));
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const int key = min(kb * 32 + 8 * (v / 4) + 4 * h + v % 4, a.kv_len - 1);
@@ -290,9 +308,9 @@ __global__ __launch_bounds__(512, 2) void flash_split_kernel(FlashArgs a) {
 #pragma unroll
         for (int d = 0; d < ND; d++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) pp[(d * 16 + v) * 64 + lane] = o[d][v];
+            for (int v = 0; v < 16; v++) pp[(d * 16 + v) * 64 + lane] = o[d][v] * unscale;
         pp[HD * 32 + lane] = m_run;
-        pp[HD * 32 + 64 + lane] = l_run;
+        pp[HD * 32 + 64 + lane] = l_run * unscale;
         return;
     }
     if (qw + lr >= a.T) return;

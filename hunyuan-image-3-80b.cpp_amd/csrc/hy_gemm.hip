@@ -7,7 +7,8 @@
 // Infinities and NaNs have no such split (inf - inf), and a value that rounds up to
 // infinity in bf16 neither: a wave whose accumulators hold a non-finite value after its
 // k-range computes that range again on the fp32 matrix cores (segment_f32), so such
-// inputs give what the fp32 product gives.
+// inputs give what the fp32 product gives.  So does a work group that met an operand too
+// small for an exact split (most of them below 2^-110).
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
 #include "hy_lds.hpp"
@@ -71,6 +72,7 @@ template <int MT>
 __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
     using L = SkLds<MT>;
     __shared__ __attribute__((aligned(16))) uint8_t abuf[2][L::BYTES];
+    __shared__ int lost_at;  // first unit of the last range that held an inexact split
     const int tid = threadIdx.x, lane = tid % WAVE, wv = tid / WAVE;
     const int lr = lane % 32, h = lane / 32;
     const int M = p.M, N = p.N, K = p.K;
@@ -86,18 +88,26 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
 
     // stages [s0, s1) of tile t on the fp32 matrix cores (non-finite operands)
     auto segment_f32 = [&](int t, int s0, int s1, v16f_t (&acc)[MT]) {
-        const float* w = p.W + (size_t)min(t * SK_BN + 32 * wv + lr, N - 1) * K + h;
+        const float* w = p.W + (size_t)min(t * SK_BN + 32 * wv + lr, N - 1) * K + 4 * h;
+        const float* arow[MT];
 #pragma unroll
-        for (int i = 0; i < MT; i++) acc[i] = v16f_t{};
-        for (int k = s0 * SK_KC; k < s1 * SK_KC; k += 2) {
-            const float b = w[k];
+        for (int i = 0; i < MT; i++) {
+            arow[i] = p.A + (size_t)min(32 * i + lr, M - 1) * K + 4 * h;
+            acc[i] = v16f_t{};
+        }
+        for (int k = s0 * SK_KC; k < s1 * SK_KC; k += 8) {
+            const v4f_t b = *reinterpret_cast<const v4f_t*>(w + k);
 #pragma unroll
-            for (int i = 0; i < MT; i++)
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.A[(size_t)min(32 * i + lr, M - 1) * K + k + h], b,
-                                                              acc[i], 0, 0, 0);
+            for (int i = 0; i < MT; i++) {
+                const v4f_t a = *reinterpret_cast<const v4f_t*>(arow[i] + k);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc[i], 0, 0, 0);
+            }
         }
     };
-    auto segment = [&](int t, int s0, int s1, v16f_t (&acc)[MT]) {
+    if (tid == 0) lost_at = -1;
+    auto segment = [&](int u, int t, int s0, int s1, v16f_t (&acc)[MT]) {
+        uint32_t lost = 0;
         const float* w = p.W + (size_t)min(t * SK_BN + 32 * wv + lr, N - 1) * K + 4 * h;
         v4f_t wb[SK_D][4];  // [stage][2 u + q]: floats 16 u + 8 q + 4 h .. + 3
         v4f_t ab[MT];
@@ -128,7 +138,8 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
             // finished before the barrier of stage s - 1
             static_for<MT>([&](auto ic) {
                 constexpr int I = decltype(ic)::value;
-                const Split2 x = split2(sgn * ab[I][0], sgn * ab[I][1]), y = split2(sgn * ab[I][2], sgn * ab[I][3]);
+                const Split2 x = split2(sgn * ab[I][0], sgn * ab[I][1], lost),
+                             y = split2(sgn * ab[I][2], sgn * ab[I][3], lost);
                 static_for<3>([&](auto qc) {
                     constexpr int Q = decltype(qc)::value;
                     lds_st64_at<BUF + Q * L::PIECE + I * 512>(a_dst, x.p[Q], y.p[Q]);
@@ -152,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const v4f_t v = wb[D][2 * UU + j / 2];
-                    const Split2 x = split2(v[2 * (j % 2)], v[2 * (j % 2) + 1]);
+                    const Split2 x = split2(v[2 * (j % 2)], v[2 * (j % 2) + 1], lost);
 #pragma unroll
                     for (int q = 0; q < 3; q++) wf[q][j] = (int)x.p[q];
                 }
@@ -182,8 +193,9 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
         for (int i = 0; i < MT; i++)
 #pragma unroll
             for (int v = 0; v < 16; v++) bad |= non_finite(acc[i][v]);
-        if (__any(bad)) segment_f32(t, s0, s1, acc);
-        __builtin_amdgcn_s_barrier();  // every wave is done with the A stages
+        if (lost_bits(lost)) lost_at = u;
+        __syncthreads();  // every wave is done with the A stages; the next write follows a later barrier
+        if (__any(bad) || lost_at == u) segment_f32(t, s0, s1, acc);
     };
 
     v16f_t acc[MT];
@@ -206,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(GemmSmallArgs p) {
     const int lo = gs_lo(p, g), hi = gs_lo(p, g + 1);
     for (int u = lo; u < hi;) {
         const int t = u / nst, s0 = u - t * nst, s1 = min(nst, s0 + (hi - u));
-        segment(t, s0, s1, acc);
+        segment(u, t, s0, s1, acc);
         if (s0 == 0 && s1 == nst) {
             store(t);
         } else {
@@ -351,6 +363,7 @@ template <int MT>
 __global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmSplitArgs p) {
     using L = GsLds<MT>;
     __shared__ __attribute__((aligned(1024))) uint8_t buf[2][L::BYTES];
+    __shared__ int lost_at;  // first unit of the last range that held an inexact split
     const int tid = threadIdx.x, lane = tid % WAVE;
     const int wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int wm = wv / 4, wn = wv % 4;  // waves w and w + 4 share a SIMD: one of each wm
@@ -373,21 +386,28 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmSplitArgs
     auto segment_f32 = [&](int m0, int n0, int s0, int s1, v16f_t (&acc)[MT][2]) {
         const float* w[2];
 #pragma unroll
-        for (int j = 0; j < 2; j++) w[j] = p.W + (size_t)min(n0 + 64 * wn + 32 * j + lr, N - 1) * K + h;
+        for (int j = 0; j < 2; j++) w[j] = p.W + (size_t)min(n0 + 64 * wn + 32 * j + lr, N - 1) * K + 4 * h;
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
             for (int j = 0; j < 2; j++) acc[i][j] = v16f_t{};
-        for (int k = s0 * GS_KC; k < s1 * GS_KC; k += 2)
+        for (int k = s0 * GS_KC; k < s1 * GS_KC; k += 8) {
+            const v4f_t b[2] = {*reinterpret_cast<const v4f_t*>(w[0] + k), *reinterpret_cast<const v4f_t*>(w[1] + k)};
 #pragma unroll
             for (int i = 0; i < MT; i++) {
-                const float a = p.A[(size_t)min(m0 + 32 * (2 * i + wm) + lr, M - 1) * K + k + h];
+                const v4f_t a = *reinterpret_cast<const v4f_t*>(
+                    p.A + (size_t)min(m0 + 32 * (2 * i + wm) + lr, M - 1) * K + k + 4 * h);
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w[j][k], acc[i][j], 0, 0, 0);
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c], b[j][c], acc[i][j], 0, 0, 0);
             }
+        }
     };
-    auto segment = [&](int m0, int n0, int s0, int s1, v16f_t (&acc)[MT][2]) {
+    if (tid == 0) lost_at = -1;
+    auto segment = [&](int u, int m0, int n0, int s0, int s1, v16f_t (&acc)[MT][2]) {
+        uint32_t lost = 0;
         const uint8_t* const ab = reinterpret_cast<const uint8_t*>(p.A + (size_t)m0 * K);
         const uint8_t* const wb = reinterpret_cast<const uint8_t*>(p.W + (size_t)n0 * K);
         uint32_t off[L::NC];
@@ -407,7 +427,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmSplitArgs
             constexpr int F = decltype(fc)::value, B = decltype(bc)::value;
             if (F == L::NA - 1 && !a_last) return;
             if constexpr (F < L::NA) x[F] *= turn_sign<GS_TURN>(s - s0);
-            const Split2 a = split2(x[F][0], x[F][1]), b = split2(x[F][2], x[F][3]);
+            const Split2 a = split2(x[F][0], x[F][1], lost), b = split2(x[F][2], x[F][3], lost);
 #pragma unroll
             for (int q = 0; q < 3; q++) {
                 uint8_t* d = F < L::NA ? wr_a + B * L::BYTES + q * L::PIECE_A + F * 2048
@@ -494,7 +514,9 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmSplitArgs
             for (int j = 0; j < 2; j++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) bad |= non_finite(acc[i][j][v]);
-        if (__any(bad)) segment_f32(m0, n0, s0, s1, acc);
+        if (lost_bits(lost)) lost_at = u;
+        __syncthreads();  // the next write follows a later barrier
+        if (__any(bad) || lost_at == u) segment_f32(m0, n0, s0, s1, acc);
     };
 
     v16f_t acc[MT][2];
@@ -525,7 +547,7 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmSplitArgs
         const int t = u / nst, s0 = u - t * nst, s1 = min(nst, s0 + (hi - u));
         int m, n;
         gs_tile(p, t, m, n);
-        segment(m * p.bm, n * GS_BN, s0, s1, acc);
+        segment(u, m * p.bm, n * GS_BN, s0, s1, acc);
         if (s0 == 0 && s1 == nst) {
             store(m * p.bm, n * GS_BN);
         } else {

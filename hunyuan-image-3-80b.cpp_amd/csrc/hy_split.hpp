@@ -16,8 +16,10 @@
 // out the rest.  So the accumulators hold the sum and its negative in turns (flip_at),
 // with the pieces of A negated alike, and the mean cancels.
 //
-// The split is exact down to 2^-110; below that the last pieces run out of exponent, an
-// absolute error of at most 2^-134 of the operand.
+// The split is exact down to 2^-110, and below wherever the last pieces' bits end at bf16's
+// smallest denormal, 2^-133 (zeros, values that were bf16 or fp16 before).  Any other
+// operand leaves a remainder that is no bf16 value, which split2 records: its users compute
+// such products on the fp32 matrix cores instead.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -51,7 +53,11 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
     const v2f_t f = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, v2bf_t));
 }
-__device__ __forceinline__ Split2 split2(float a, float b) {
+// lost gathers the last remainders' bits; lost_bits(lost) once a split was not exact (a bf16
+// value has the low half of its fp32 bits clear): one operation for two operands, eleven
+// for their split
+__device__ __forceinline__ bool lost_bits(uint32_t lost) { return (lost & 0xffffu) != 0; }
+__device__ __forceinline__ Split2 split2(float a, float b, uint32_t& lost) {
     Split2 s;
     s.p[0] = pk_bf16(a, b);
     a -= __uint_as_float(s.p[0] << 16);
@@ -60,6 +66,8 @@ __device__ __forceinline__ Split2 split2(float a, float b) {
     a -= __uint_as_float(s.p[1] << 16);
     b -= __uint_as_float(s.p[1] & 0xffff0000u);
     s.p[2] = pk_bf16(a, b);
+    lost |= __float_as_uint(a) | __float_as_uint(b);
+    asm("" : "+v"(lost));  // formed here: the compiler would gather many remainders first, in registers
     return s;
 }
 __device__ __forceinline__ v16f_t mfma_bf16(v4i_t a, v4i_t b, v16f_t c) {

@@ -147,8 +147,10 @@ int hy_model_forward_hidden(hy_model_ctx* ctx, const float* inputs_embeds_dev, u
 
 /* lm_head_f32 (src/hunyuan_full_model.cpp:298-318) and the projections' GEMM:
  * out[t][v] = sum_h x[t][h] * w[v][h] (+ resid[t][v] when resid_dev is not NULL), in
- * fp32 (fp32 MFMA, or exact three-way bf16 splits of the operands); x [T][hidden], w [vocab][hidden], all device memory; hidden a multiple
- * of 16.  Mid-size shapes split the reduction over a per-device scratch that the
+ * fp32: fp32 FMAs and MFMAs, or six products of three-way bf16 splits of the operands
+ * where these are exact (every value from 2^-110 to 2^127, and smaller ones whose bits
+ * end at 2^-133; other values are multiplied by fp32 MFMAs).  x [T][hidden], w
+ * [vocab][hidden], all device memory; hidden a multiple of 16.  Mid-size shapes split the reduction over a per-device scratch that the
  * library allocates on first use and orders between calls with an event: those shapes
  * return HY_ERR_UNSUPPORTED under stream capture (hy_model_forward, whose context
  * owns its scratch, can be captured). */

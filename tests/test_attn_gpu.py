@@ -358,3 +358,64 @@ def test_prompt_values_without_a_split(gpu):
     out = m.run(x)
     assert np.isfinite(out[:32]).all() and not np.isfinite(out[40:]).any()
     m.close()
+
+
+@pytest.mark.parametrize("shp", SHAPES, ids=["hd64", "hd128"])
+@pytest.mark.parametrize("e", [-112, -118, -124])
+def test_prompt_tiny_operands(gpu, shp, e):
+    """Keys, queries and values below 2^-110, which three bf16 pieces do not hold, keep fp32's
+    accuracy (test_prompt_tiles' bound); T = 300 cuts tiles into chunks."""
+    nh, nkv, hd = shp["nh"], shp["nkv"], shp["hd"]
+    nq, nk = nh * hd, nkv * hd
+    for T, which in ((90, "k"), (90, "q"), (90, "v"), (300, "v")):
+        m, w = _ctx(gpu, shp, max_tokens=T, seed=5)
+        qkv, o_w, q_norm, k_norm = w.qkv_w.copy(), w.o_w, w.q_norm, w.k_norm
+        if which == "v":
+            qkv[nq + nk:] = np.ldexp(qkv[nq + nk:], e)
+            o_w = np.ldexp(o_w, 60)
+        else:
+            s = 1 if which == "q" else -1
+            q_norm, k_norm = np.ldexp(q_norm, s * e), np.ldexp(k_norm, -s * e)
+        m.upload(qkv, o_w, q_norm, k_norm)
+        x = np.random.default_rng(T).standard_normal((T, shp["H"])).astype(np.float32)
+        out, dq, dk, dv = m.run(x, debug=True)
+        q, k, v = dq.reshape(T, nh, hd), dk.reshape(T, nkv, hd), dv.reshape(T, nkv, hd)
+        ref = _attn64(q, k, v, nh, nkv) @ o_w.astype(np.float64).T
+        assert np.linalg.norm(out - ref) <= 1e-5 * np.linalg.norm(ref), (which, T)
+        m.close()
+
+
+@pytest.mark.parametrize("shp", SHAPES, ids=["hd64", "hd128"])
+def test_prompt_tiny_probabilities(gpu, shp):
+    """A value of 2^90 under a probability of 2^-125 .. 2^-118 keeps the probability's
+    accuracy.  Bound: the base-2 scores, up to some hundreds, carry rounding errors of 2^-24
+    of themselves, which the exponential makes relative ones (below 3e-5); pieces of the
+    probability itself would end at 2^-133 and leave 1e-4 to 2e-3."""
+    T, nh, nkv, hd = 200, shp["nh"], shp["nkv"], shp["hd"]
+    m, w = _ctx(gpu, shp, max_tokens=T, seed=7)
+    nq, nk = nh * hd, nkv * hd
+    qkv = w.qkv_w.copy()
+    qkv[:, 0] = 0.0
+    qkv[nq + nk + 5, :] = 0.0
+    qkv[nq + nk + 5, 0] = 1.0  # dim 5 of the first value head is x[:, 0] itself
+    o_w = np.zeros_like(w.o_w)
+    o_w[:, 5] = 1.0  # the output: that dim of the first head
+    # base-2 score differences of 120 are among the larger ones
+    q_norm = (w.q_norm * np.float32(24.0 * np.sqrt(64.0 / hd))).astype(np.float32)
+    m.upload(qkv, o_w, q_norm, w.k_norm)
+    x = np.random.default_rng(7).standard_normal((T, shp["H"])).astype(np.float32)
+    x[:, 0] = 0.0
+    out, dq, dk, dv = m.run(x, debug=True)
+    q, k = dq.reshape(T, nh, hd)[:, 0].astype(np.float64), dk.reshape(T, nkv, hd)[:, 0].astype(np.float64)
+    s = q @ k.T / np.sqrt(hd)
+    s[np.triu_indices(T, 1)] = -np.inf
+    p = np.exp(s - s.max(axis=1, keepdims=True))
+    hit = (p > 2.0 ** -125) & (p < 2.0 ** -118)
+    j = int(hit.sum(axis=0).argmax())  # the key with most of them
+    t = np.flatnonzero(hit[:, j])
+    assert t.size >= 3
+    x[j, 0] = np.float32(2.0 ** 90)
+    out = m.run(x)
+    want = (p[:, j] / p.sum(axis=1))[t] * 2.0 ** 90
+    assert np.sqrt(np.mean((out[t, 0] / want - 1.0) ** 2)) <= 3e-5
+    m.close()

@@ -106,3 +106,38 @@ def test_nine_to_sixteen_rows(gpu, M, N, K):
     check(gpu.lm_head_f32(x, w, r), x, w, r)
     # a row's bits do not depend on how many rows share the pass
     assert np.array_equal(got[:8].view(np.uint32), gpu.lm_head_f32(x[:8], w).view(np.uint32))
+
+
+# small-batch tiles of every height, cut and whole, and the larger kernel with and without
+# scratch
+@pytest.mark.parametrize("e", [-104, -109, -112, -116, -124, -134, -146])
+@pytest.mark.parametrize("M,N,K", [(20, 300, 512), (48, 2048, 1024), (90, 257, 256), (128, 517, 512),
+                                   (300, 6144, 512), (300, 33000, 48)])
+def test_operands_without_an_exact_split(gpu, M, N, K, e):
+    """Below 2^-110 three bf16 pieces do not hold an fp32 value: rows of such values, on either
+    side, keep fp32's accuracy (6e-7 of a row's norm measured; unmended pieces leave 2e-6 at
+    2^-116 and 5e-4 at 2^-124).  Their neighbours, and sums that mix both, too."""
+    rng = np.random.default_rng(-e)
+
+    def tiny(*shape):
+        return np.ldexp(rng.standard_normal(shape), e).astype(np.float32)
+
+    def rel(got, x, w):
+        ref = x.astype(np.float64) @ w.astype(np.float64).T
+        return (np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)).max()
+
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    w = np.ldexp(rng.standard_normal((N, K)), 60).astype(np.float32)
+    x[M // 2:] = tiny(M - M // 2, K)
+    got = gpu.lm_head_f32(x, w)
+    assert rel(got[:M // 2], x[:M // 2], w) <= 1.5e-6
+    assert rel(got[M // 2:], x[M // 2:], w) <= 1.5e-6
+    x = np.ldexp(rng.standard_normal((M, K)), 60).astype(np.float32)
+    w = tiny(N, K)
+    w[0] = 0.0
+    got = gpu.lm_head_f32(x, w)
+    assert rel(got, x, w) <= 1.5e-6 and not got[:, 0].any()
+    # a single such operand that carries its row: 2^60 against zeros
+    x[:] = 0.0
+    x[:, K - 1] = np.float32(2.0 ** 60)
+    assert np.array_equal(gpu.lm_head_f32(x, w), np.ldexp(w[:, K - 1], 60)[None].repeat(M, 0))
