@@ -114,11 +114,20 @@ __device__ __forceinline__ int operand_lane_off(int lr, int lg) { return lr * 32
 // 16-31) nibbles of the row's 16 stored bytes; lanes 2j and 2j + 1 read the same
 // nibble row.  nib = the chunk's nibble rows + 16 * (l / 2), dst = its int8 rows + 16 l,
 // sh = 4 - 4 h (the same for rows l / 2 and 32 + l / 2).
+//
+// PLAIN: mask and sign flip as two operations with literals.  As one three-input operation
+// they need the mask in a register, and the wide shape has none: a copy's address was
+// spilled, and its reload in the stage loop waited for the copies in flight.  A layer of
+// H 4096, I 3072, E 16, K 4 at T = 400: 345 us, with the spill 368 (gate/up alone 233, and
+// 217 with the five operations that leave n - 8 itself); E 64, K 8 at T = 800 928 and 969,
+// at T = 4096 3.77 and 3.86 ms.  The tall shape has registers left and takes the one
+// operation less (T = 300: 550 us a layer with either).
+template <bool PLAIN>
 __device__ __forceinline__ void unpack_q4_chunk_at(uint32_t nib, uint32_t dst, uint32_t sh) {
     v4i_t w0 = lds_b128_at<0>(nib);
     v4i_t w1 = lds_b128_at<512>(nib);
     lds_wait(w0, w1);
-    auto cv = [sh](int v) { return unpack_q4x16(v, sh); };
+    auto cv = [sh](int v) { return unpack_q4x16<PLAIN>(v, sh); };
     lds_st128_at<0>(dst, v4i_t{cv(w0[0]), cv(w0[1]), cv(w0[2]), cv(w0[3])});
     lds_st128_at<1024>(dst, v4i_t{cv(w1[0]), cv(w1[1]), cv(w1[2]), cv(w1[3])});
 }
@@ -468,7 +477,7 @@ __global__ __launch_bounds__(SH::THREADS, SH::WG_PER_CU) void moe_mfma_kernel(Mm
             // aun[s & 1], last read by stage s - 2's math, which every wave finished before
             // the previous barrier
             const uint32_t ab = (uint32_t)((s & 1) * SH::ST_A);
-            unpack_q4_chunk_at(un_src + soff, un_dst + ab, un_sh);
+            unpack_q4_chunk_at<TT == 2>(un_src + soff, un_dst + ab, un_sh);
             lds_wait();
             abase = aun0 + ab + a_lane;
         } else {
@@ -576,8 +585,8 @@ __global__ __launch_bounds__(WAVE) void block_dots_mfma_kernel(const uint8_t* __
         lds_st128(nib_s + lane * 16, r < rows ? dw4(wq) : zero4);
         lds_wait();
         __syncthreads();
-        unpack_q4_chunk_at(lds_off(nib_s) + (uint32_t)((lane >> 1) * 16), lds_off(a_s) + (uint32_t)(lane * 16),
-                           unpack_q4_shift(lane));
+        unpack_q4_chunk_at<false>(lds_off(nib_s) + (uint32_t)((lane >> 1) * 16), lds_off(a_s) + (uint32_t)(lane * 16),
+                                  unpack_q4_shift(lane));
     } else {
         lds_st128(a_s + lane * 32 + swz_half(lane, 0), r < rows ? dw4(wq) : zero4);
         lds_st128(a_s + lane * 32 + swz_half(lane, 1), r < rows ? dw4(wq + 16) : zero4);

@@ -37,8 +37,11 @@ struct MmArgs {
 // from denormals) -- and the epilogue multiplies by 1/16.  Against n - 8 itself (five
 // operations per four weights): Q4_0 layers of T = 48 465 -> 454 us, 4096 skewed tokens
 // 3.94 -> 3.92 ms, a decoder layer of T = 300 906 -> 895 us (same box).
+template <bool PLAIN = false>
 __device__ __forceinline__ int unpack_q4x16(int v, uint32_t sh) {
-    return (int)((((uint32_t)v << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
+    uint32_t n = ((uint32_t)v << sh) & 0xF0F0F0F0u;
+    if constexpr (PLAIN) asm("" : "+v"(n));  // keeps the two operations apart
+    return (int)(n ^ 0x80808080u);
 }
 
 // The exact int32 dots of one 32-wide GGUF block over a 32x32 tile (K = 32 is one
