@@ -14,6 +14,7 @@
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
 #include "hy_layout.hpp"
+#include "hy_rules.hpp"
 #include "../host/hy_gguf.hpp"
 
 namespace {
@@ -193,21 +194,6 @@ int tile_bound_routed(int T, int K, int E, int NT) {
 // moe_forward_cpu (src/attention.cpp:268-275), which renormalise at every K.
 int renorm_rule(int32_t norm, uint32_t K) { return (norm == HY_NORM_ALWAYS || (norm != HY_NORM_OFF && K > 1)) ? 1 : 0; }
 
-// largest batch the one-launch decode routing takes; the decode GEMV takes at least
-// these in AUTO mode
-constexpr uint32_t kGemvMaxTokens = 16;
-
-// AUTO mode: the decode GEMV or the MFMA grouped GEMM.  Measured crossover on one MI355X
-// (H 4096, I 3072, E 64, K 8): Q4_0 GEMV 304 vs MFMA 318 us at T=24, 361 vs 314 at T=32 (up
-// to ~3 pairs per expert); Q8_0 400 vs 405 us at T=16, 470 vs 426 at T=24 (~2).
-bool gemv_batch(int wt, uint32_t T, int K, int E) {
-    if (T <= kGemvMaxTokens) return true;
-    const uint64_t pairs = (uint64_t)T * (uint64_t)K;
-    if (wt == HY_TYPE_Q4_0) return pairs <= 3ull * (uint64_t)E;
-    if (wt == HY_TYPE_Q8_0) return pairs <= 2ull * (uint64_t)E;
-    return false;
-}
-
 int check_cfg(const hy_moe_config* c) {
     if (!c) return fail(HY_ERR_INVALID, "null config");
     if (c->hidden == 0 || c->hidden % 64)
@@ -298,7 +284,7 @@ int forward_impl(hy_moe_ctx* c, uint32_t layer, const float* x, uint32_t T, floa
     const bool mfma_fits = (uint64_t)T * (uint64_t)(K + 1) * (uint64_t)H < (1ull << 32) &&
                            (uint64_t)T * (uint64_t)(K + 1) * (uint64_t)I < (1ull << 32);
     const bool mfma = c->path != HY_PATH_VALU && hy::mfma_path_ok(wt, H, I) && mfma_fits &&
-                      (c->path == HY_PATH_MFMA || !gemv_batch(wt, T, K, E));
+                      (c->path == HY_PATH_MFMA || !hy::gemv_batch(wt, T, K, E, H, I, has_shared));
     const int shape = mfma ? hy::mfma_shape(wt, iT, K, E, H, I) : -1;
     const bool mfma32 = c->path == HY_PATH_AUTO && wt == HY_TYPE_F32 && hy::mfma_f32_ok(iT, K, E, H, I);
     const int NT = mfma     ? hy::mfma_shape_tokens(shape)
@@ -314,7 +300,7 @@ int forward_impl(hy_moe_ctx* c, uint32_t layer, const float* x, uint32_t T, floa
         HY_TRY(timed(c, hy::KID_ROUTER, s, [&] {
             return hy::launch_decode_logits(x, L.router, H, E, c->logits, prequant ? nullptr : c->xq, c->xd, c->xs, s);
         }));
-    } else if (!ext && !mfma && wt != HY_TYPE_F32 && T <= kGemvMaxTokens && iT * K <= hy::MAX_DECODE_PAIRS) {
+    } else if (!ext && !mfma && wt != HY_TYPE_F32 && T <= hy::GEMV_MAX_TOKENS && iT * K <= hy::MAX_DECODE_PAIRS) {
         // decode: router logits, then top-k, dispatch lists and Q8_0 of x in one launch
         HY_TRY(timed(c, hy::KID_ROUTER, s, [&] {
             return hy::launch_route_decode(x, L.router, iT, H, E, K, renorm,
