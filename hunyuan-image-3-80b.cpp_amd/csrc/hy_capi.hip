@@ -285,7 +285,7 @@ int forward_impl(hy_moe_ctx* c, uint32_t layer, const float* x, uint32_t T, floa
                            (uint64_t)T * (uint64_t)(K + 1) * (uint64_t)I < (1ull << 32);
     const bool mfma = c->path != HY_PATH_VALU && hy::mfma_path_ok(wt, H, I) && mfma_fits &&
                       (c->path == HY_PATH_MFMA || !hy::gemv_batch(wt, T, K, E, H, I, has_shared));
-    const int shape = mfma ? hy::mfma_shape(wt, iT, K, E, H, I) : -1;
+    const int shape = mfma ? hy::mfma_shape(wt, iT, K, E, H, I, has_shared) : -1;
     const bool mfma32 = c->path == HY_PATH_AUTO && wt == HY_TYPE_F32 && hy::mfma_f32_ok(iT, K, E, H, I);
     const int NT = mfma     ? hy::mfma_shape_tokens(shape)
                    : mfma32 ? hy::mfma_f32_tokens(iT, K, E)

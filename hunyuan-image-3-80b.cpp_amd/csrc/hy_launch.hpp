@@ -97,7 +97,7 @@ bool mfma_path_ok(int wtype, int H, int I);
 // tile shape of the MFMA path for this batch, and its pairs per tile (the dispatch
 // must tile with it)
 enum MfmaShape { MM_SHAPE_WIDE = 0, MM_SHAPE_TALL = 1, MM_SHAPE_FEW = 2 };
-int mfma_shape(int wtype, int T, int K, int E, int H, int I);
+int mfma_shape(int wtype, int T, int K, int E, int H, int I, int has_shared);
 int mfma_shape_tokens(int shape);
 // the grouped GEMM's work counters (ints of device memory a caller keeps per context);
 // launch_gather_act zeroes them for the gate/up and down launches that follow it

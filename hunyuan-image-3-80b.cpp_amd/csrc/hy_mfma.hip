@@ -47,6 +47,7 @@
 #include "hy_layout.hpp"
 #include "hy_lds.hpp"
 #include "hy_mfma.hpp"
+#include "hy_rules.hpp"
 
 namespace hy {
 
@@ -653,18 +654,14 @@ bool mfma_path_ok(int wtype, int H, int I) {
     return (wtype == HY_TYPE_Q8_0 || wtype == HY_TYPE_Q4_0) && shape_fits<ShapeWide>(H, I);
 }
 
-// The stream of hy_mfma_few.hip wins while most experts fit one of its 32-pair tiles, as a
-// second tile streams the weights again: H 4096, I 3072, E 64, K 8, few against tall: T = 208
-// (26 pairs per expert) Q4_0 381 / 483 us, Q8_0 533 / 578; T = 240 444 / 494 and 640 / 592.
-// Where the gate/up weights fit the Infinity Cache a second tile finds them there: H 2048,
-// I 1536, E 16, K 4: T = 200 (50 pairs) Q4_0 90 / 115, Q8_0 95 / 109; T = 300 102 / 129
-// and 104 / 123.  The tall shape (64-pair tiles, 256-row blocks) wins while experts see
-// about 64 pairs each (a 128-pair tile would leave half its waves idle); beyond ~96 the
-// wide shape's reuse of every weight byte over 128 pairs wins.
-int mfma_shape(int wtype, int T, int K, int E, int H, int I) {
+// The stream of hy_mfma_few.hip while experts see few pairs (few_batch).  Then the tall
+// shape (64-pair tiles, 256-row blocks) wins while experts see about 64 pairs each (a
+// 128-pair tile would leave half its waves idle); beyond ~96 the wide shape's reuse of every
+// weight byte over 128 pairs wins.
+int mfma_shape(int wtype, int T, int K, int E, int H, int I, int has_shared) {
     const int64_t pairs = (int64_t)T * K;
     const bool cached = (size_t)(E + 1) * 2 * I * (H / QK) * block_bytes(wtype) <= INFINITY_CACHE;
-    if (pairs <= (int64_t)(cached ? 64 : 26) * E) return MM_SHAPE_FEW;
+    if (few_batch(wtype, T, K, E, I, has_shared, cached)) return MM_SHAPE_FEW;
     const bool tall = shape_fits<ShapeTall>(H, I) && pairs < (int64_t)96 * E;
     return tall ? MM_SHAPE_TALL : MM_SHAPE_WIDE;
 }

@@ -42,4 +42,29 @@ inline bool gemv_batch(int wt, uint32_t T, int K, int E, int H, int I, int has_s
     return passes / mats * (ring ? 1 : 2) <= (q4 ? 0.95 + 750.0 / waves : 0.65 + 700.0 / waves);
 }
 
+// The grouped GEMM's batches that the stream of hy_mfma_few.hip takes (cached: its
+// gate/up weights fit the Infinity Cache).
+//
+// It wins while most experts fit one of its 32-pair tiles, as a second tile streams the weights
+// again.  H 4096, I 3072, E 64, K 8, stream against the tall shape: T = 208 (26 pairs per
+// expert) Q4_0 381 / 483 us, Q8_0 533 / 578; T = 240 444 / 494 and 640 / 592.  (Q4_0 alone would
+// cross past 30 pairs; one line serves both.)  Where the weights are cached a second tile finds
+// them there: up to 64 pairs, past which the tall shape too has a second tile.  Q8_0 between 32
+// and 60 pairs, where evenly routed experts fill two of the stream's tiles and one of the tall
+// shape's, gains only while the stream's waves leave the chip idle (3 per SIMD are resident,
+// the line is at nine tenths): E 16, K 4, 2048 x 1536 T = 200 (1880 waves) 93 / 110, E 8, K 1,
+// 4096 x 3072 T = 400 (2690) 175 / 188; with more E 32, K 4, 2048 x 1536 T = 300 (2980)
+// 155 / 136, T = 448 158 / 137, but T = 496 165 / 164; E 64, K 8, 1024 x 768 T = 400 (3460)
+// 105 / 92, T = 496 109 / 110.  (Skewed routing gains from the stream at these sizes too,
+// 145 / 169 and 90 / 95 at T = 400; the rule goes by even routing.)  Q4_0, with half the bytes,
+// gains throughout: E 32, K 4, 2048 x 1536 T = 400 127 / 134, E 64, K 8, 1024 x 768 90 / 95.
+inline bool few_batch(int wt, int64_t T, int K, int E, int I, int has_shared, bool cached) {
+    const int64_t pairs = T * K;
+    if (pairs <= 26 * (int64_t)E) return true;
+    if (!cached || pairs > 64 * (int64_t)E) return false;
+    if (wt == HY_TYPE_Q4_0 || pairs <= 32 * (int64_t)E || pairs > 60 * (int64_t)E) return true;
+    const int64_t tiles = pairs / 32 + E / 2 + (has_shared ? T / 32 : 0);  // half an expert's last tile empty
+    return tiles * (2 * I / 64) <= 1024 * 3 * 9 / 10;
+}
+
 }  // namespace hy

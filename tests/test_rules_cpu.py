@@ -12,6 +12,9 @@ SHIM = """
 extern "C" int gemv_batch(int wt, unsigned T, int K, int E, int H, int I, int sh) {
     return hy::gemv_batch(wt, T, K, E, H, I, sh);
 }
+extern "C" int few_batch(int wt, int T, int K, int E, int I, int sh, int cached) {
+    return hy::few_batch(wt, T, K, E, I, sh, cached != 0);
+}
 """
 Q4, Q8 = 2, 8
 
@@ -73,3 +76,37 @@ def test_gemv_line_ends(rules):
             assert not rules.gemv_batch(Q4, 5 * E + 17, K, E, 4096, 3072, sh)
             assert not rules.gemv_batch(Q8, 5 * E + 17, K, E, 4096, 3072, sh)
             assert not rules.gemv_batch(0, 17, K, E, 4096, 3072, sh)
+
+
+# type, E, K, H, I (weights in the Infinity Cache): (T, stream, tall shape)
+FEW_TIMES = [
+    (Q4, 32, 4, 2048, 1536, (256, 99, 130), (400, 127, 134), (512, 149, 172)),
+    (Q4, 64, 8, 1024, 768, (300, 77, 94), (400, 90, 95), (512, 97, 115)),
+    (Q4, 16, 4, 4096, 3072, (200, 212, 220), (256, 242, 288)),
+    (Q8, 16, 4, 2048, 1536, (150, 91, 108), (200, 93, 110), (256, 105, 113)),
+    (Q8, 32, 4, 2048, 1536, (256, 132, 133), (300, 155, 136), (400, 157, 137), (448, 158, 138), (496, 165, 164)),
+    (Q8, 32, 4, 1024, 1408, (256, 78, 88), (300, 89, 88), (400, 100, 91), (496, 102, 108)),
+    (Q8, 32, 4, 1024, 768, (300, 69, 74), (400, 72, 75), (512, 82, 83)),
+    (Q8, 64, 8, 1024, 768, (256, 87, 89), (300, 92, 92), (400, 105, 93), (448, 107, 94), (496, 109, 110)),
+    (Q8, 48, 6, 1536, 1024, (270, 104, 106), (400, 116, 108), (448, 118, 110), (496, 123, 132)),
+    (Q8, 64, 8, 1024, 1408, (256, 121, 129), (300, 135, 131), (400, 153, 137), (448, 156, 138)),
+    (Q8, 8, 1, 4096, 3072, (256, 149, 180), (300, 174, 183), (400, 175, 188)),
+    (Q8, 8, 2, 4096, 3072, (150, 150, 178), (200, 169, 180), (256, 171, 186)),
+    (Q8, 16, 2, 2048, 1536, (300, 90, 110), (400, 104, 112), (512, 103, 113)),
+]
+
+
+@pytest.mark.parametrize("row", FEW_TIMES, ids=lambda r: "-".join(map(str, r[:5])))
+def test_stream_or_tall(rules, row):
+    wt, E, K, H, I = row[:5]
+    for T, few, tall in row[5:]:
+        took = few if rules.few_batch(wt, T, K, E, I, 1, 1) else tall
+        assert took <= 1.05 * min(few, tall), T
+
+
+def test_stream_line_without_the_cache(rules):
+    for wt in (Q4, Q8):
+        for E, K in ((64, 8), (16, 4)):
+            T = 26 * E // K
+            assert rules.few_batch(wt, T, K, E, 3072, 1, 0) and not rules.few_batch(wt, T + 1, K, E, 3072, 1, 0)
+            assert not rules.few_batch(wt, 64 * E // K + 1, K, E, 64, 0, 1)
