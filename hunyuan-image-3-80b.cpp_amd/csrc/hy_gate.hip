@@ -5,6 +5,7 @@
 // forward does not use the dense [T,E,C] representation.
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
+#include "hy_rules.hpp"
 
 namespace hy {
 
@@ -137,11 +138,10 @@ __global__ __launch_bounds__(256) void rms_norm_w_kernel(const float* __restrict
     for (int h = lane; h < H; h += WAVE) out[(size_t)row * H + h] = xr[h] * rms * w[h];
 }
 
-// The same for H a multiple of 256 up to 4096, one work group per row: every wave loads the
+// The same for H a multiple of 256 up to 4096 (norm_in_registers), one work group per row: every wave loads the
 // whole row into registers at once and forms the whole sum (the same order, so the same
 // bits), then writes every fourth chunk.  Bound: latency; one wave per row with one load in
 // flight took 30 us at T = 300, H = 4096 (this: 6).
-constexpr int RMSW_MAX_CHUNKS = 16;
 __global__ __launch_bounds__(256) void rms_norm_w_reg_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              int H, float eps, float* __restrict__ out) {
     const int row = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void rms_norm_w_reg_kernel(const float* __rest
 hipError_t launch_rms_norm_w(const float* x, const float* w, int T, int H, float eps, float* out, hipStream_t s) {
     // 16-byte rows and pointers: whatever a caller passes is aligned to its floats only
     const bool vec = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
-    if (vec && H % (4 * WAVE) == 0 && H <= 4 * WAVE * RMSW_MAX_CHUNKS)
+    if (vec && norm_in_registers(T, H))
         hipLaunchKernelGGL(rms_norm_w_reg_kernel, dim3(T), dim3(256), 0, s, x, w, H, eps, out);
     else
         hipLaunchKernelGGL(rms_norm_w_kernel, dim3((T + 3) / 4), dim3(256), 0, s, x, w, T, H, eps, out);

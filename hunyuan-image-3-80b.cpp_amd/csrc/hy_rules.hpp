@@ -67,4 +67,13 @@ inline bool few_batch(int wt, int64_t T, int K, int E, int I, int has_shared, bo
     return tiles * (2 * I / 64) <= 1024 * 3 * 9 / 10;
 }
 
+// RMSNorm rows read by four waves each, whole rows in registers (rms_norm_w_reg_kernel),
+// against one wave per row: ahead while the rows are long or few.  us, four waves / one:
+// H 4096 T = 1 6 / 11, 1000 7 / 25, 8192 40 / 59; H 1536 T = 4096 10 / 13; H 1024 T = 2000 6.4 / 6.4,
+// 4096 8.1 / 7.7; H 256 T = 2000 6.2 / 6.3, 8192 10.9 / 6.2.
+constexpr int RMSW_MAX_CHUNKS = 16;  // of 256 floats
+inline bool norm_in_registers(int T, int H) {
+    return H % 256 == 0 && H <= 256 * RMSW_MAX_CHUNKS && (H > 1024 || T <= 2048);
+}
+
 }  // namespace hy

@@ -11,6 +11,11 @@ import hy_oracle as O
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("H,T", [(256, 2048), (256, 2049), (1024, 2049), (1280, 2049), (4096, 300)])
+def test_rms_norm_w_many_rows(gpu, H, T):
+    test_rms_norm_w(gpu, H, T)
+
+
 @pytest.mark.parametrize("H", [256, 320, 2048, 4096, 4352])
 @pytest.mark.parametrize("T", [1, 5])
 def test_rms_norm_w(gpu, H, T):

@@ -15,6 +15,7 @@ extern "C" int gemv_batch(int wt, unsigned T, int K, int E, int H, int I, int sh
 extern "C" int few_batch(int wt, int T, int K, int E, int I, int sh, int cached) {
     return hy::few_batch(wt, T, K, E, I, sh, cached != 0);
 }
+extern "C" int norm_in_registers(int T, int H) { return hy::norm_in_registers(T, H); }
 """
 Q4, Q8 = 2, 8
 
@@ -110,3 +111,15 @@ def test_stream_line_without_the_cache(rules):
             T = 26 * E // K
             assert rules.few_batch(wt, T, K, E, 3072, 1, 0) and not rules.few_batch(wt, T + 1, K, E, 3072, 1, 0)
             assert not rules.few_batch(wt, 64 * E // K + 1, K, E, 64, 0, 1)
+
+
+# H, T, rows in registers, one wave per row
+@pytest.mark.parametrize("H,T,regs,wave", [(4096, 1, 6.3, 10.7), (4096, 8192, 39.7, 58.5), (2816, 300, 6.2, 9.3),
+                                           (1536, 4096, 10.2, 13.4), (1536, 8192, 17.7, 22.7), (1024, 2000, 6.4, 6.4),
+                                           (1024, 4096, 8.1, 7.7), (256, 2000, 6.2, 6.3), (256, 8192, 10.9, 6.2)])
+def test_norm_kernel(rules, H, T, regs, wave):
+    assert (regs if rules.norm_in_registers(T, H) else wave) <= 1.02 * min(regs, wave)
+
+
+def test_norm_registers_hold_the_row(rules):
+    assert not any(rules.norm_in_registers(5, H) for H in (64, 1088, 4100, 4352, 8192))
