@@ -142,8 +142,8 @@ __global__ __launch_bounds__(256) void rms_norm_w_kernel(const float* __restrict
 // whole row into registers at once and forms the whole sum (the same order, so the same
 // bits), then writes every fourth chunk.  Bound: latency; one wave per row with one load in
 // flight took 30 us at T = 300, H = 4096 (this: 6).
-__global__ __launch_bounds__(256) void rms_norm_w_reg_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                             int H, float eps, float* __restrict__ out) {
+__global__ __launch_bounds__(256) void rms_norm_w_reg_kernel(const float* x, const float* __restrict__ w, int H,
+                                                             float eps, float* out) {
     const int row = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     const int nc = H / (4 * WAVE);
     const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * H) + lane;
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256) void rms_norm_w_reg_kernel(const float* __rest
             a = fmaf(v[i].w, v[i].w, a);
         }
     const float ss = __shfl(tree_sum64(a), 0, WAVE);
-    __syncthreads();  // out may be x: no wave writes before all have read
+    __syncthreads();  // out may be x (neither is __restrict__): no wave writes before all have read
     const float rms = 1.0f / sqrtf(ss / (float)H + eps);
     const float4* wr = reinterpret_cast<const float4*>(w) + lane;
     float4* o = reinterpret_cast<float4*>(out + (size_t)row * H) + lane;

@@ -1030,9 +1030,8 @@ __global__ __launch_bounds__(256) void rms_norm_quant_kernel(const float* __rest
 // (T = 300, H = 4096: 9 us where one wave per row takes 16).
 constexpr int RMSQ_MAX_CHUNKS = 16;
 template <int WPR>
-__global__ __launch_bounds__(256) void rms_norm_quant_reg_kernel(const float* __restrict__ x,
-                                                                 const float* __restrict__ w, int T, int H, float eps,
-                                                                 float* __restrict__ xn, int8_t* __restrict__ q,
+__global__ __launch_bounds__(256) void rms_norm_quant_reg_kernel(const float* x, const float* __restrict__ w, int T,
+                                                                 int H, float eps, float* xn, int8_t* __restrict__ q,
                                                                  float* __restrict__ d, int* __restrict__ qsum) {
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     const int row = WPR == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
@@ -1053,7 +1052,7 @@ __global__ __launch_bounds__(256) void rms_norm_quant_reg_kernel(const float* __
             a = fmaf(v[i].w, v[i].w, a);
         }
     const float ss = __shfl(tree_sum64(a), 0, WAVE);
-    if (WPR == 4) __syncthreads();  // xn may be x: no wave writes before all have read
+    if (WPR == 4) __syncthreads();  // xn may be x (neither is __restrict__): no wave writes before all have read
     const float rms = 1.0f / sqrtf(ss / (float)H + eps);
     const int nb = H / QK;
 #pragma unroll

@@ -261,7 +261,7 @@ int hy_block_dots(int32_t wtype, const void* w_blocks_dev, const void* x_blocks_
                   uint32_t n, int32_t path, int32_t* out_dev, void* stream);
 
 /* RMSNorm over T rows of H: out = x * (1/sqrtf(ss/H + eps)) * w, ss in the router's
- * blocked order; w_dev may be NULL for unit weight.  rms_norm_f32
+ * blocked order; w_dev may be NULL for unit weight; out_dev may be x_dev.  rms_norm_f32
  * (src/rms_norm.cpp:9-33). */
 int hy_rms_norm(const float* x_dev, uint32_t T, uint32_t H, float eps, float* out_dev, void* stream);
 int hy_rms_norm_w(const float* x_dev, const float* w_dev, uint32_t T, uint32_t H, float eps,
