@@ -26,6 +26,7 @@
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
 #include "hy_lds.hpp"
+#include "hy_rules.hpp"
 
 namespace hy {
 
@@ -186,15 +187,9 @@ size_t gemm_nt_f32_ws_bytes(int max_rows) {
     return max(gemm_small_ws_bytes(max_rows), gemm_split_ws_bytes(max_rows));
 }
 
-// the grids of the stand-alone product that are given scratch: 64 to 1023 tiles of 128 x 128
-bool gemm_nt_f32_uses_ws(int M, int N, int K) {
-    const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-    return K % 32 == 0 && tiles >= 64 && tiles < 1024 && tiles * (K / 32) >= 2048;
-}
-
 hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                               hipStream_t s, float* ws) {
-    if (M <= 16) {
+    if (M <= GEMM_GEMV_ROWS) {
         using std::integral_constant;
         auto gemv = [&](auto mb, auto depth, auto rpw, int m0, int m) {
             constexpr int MB = decltype(mb)::value, D = decltype(depth)::value, RPW = decltype(rpw)::value;

@@ -15,6 +15,7 @@
 #include "../host/hy_gguf.hpp"
 #include "hy_device.hpp"
 #include "hy_launch.hpp"
+#include "hy_rules.hpp"
 
 namespace hy {
 int set_last_error(int code, const std::string& msg);  // hy_capi.hip
@@ -457,7 +458,7 @@ int hy_lm_head_f32(const float* x, const float* w, const float* resid, uint32_t 
         return fail(HY_ERR_INVALID, "bad GEMM shape T=%u hidden=%u vocab=%u (hidden a multiple of 16)", T, hidden,
                     vocab);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!hy::gemm_nt_f32_uses_ws((int)T, (int)vocab, (int)hidden)) {
+    if (!hy::gemm_mid_size((int)T, (int)vocab, (int)hidden)) {
         HIP_TRY(hy::launch_gemm_nt_f32(x, w, resid, out, (int)T, (int)vocab, (int)hidden, s, nullptr));
         return HY_OK;
     }
@@ -474,6 +475,10 @@ int hy_lm_head_f32(const float* x, const float* w, const float* resid, uint32_t 
         return fail(HY_ERR_UNSUPPORTED,
                     "hy_lm_head_f32 with T=%u vocab=%u uses a shared scratch and cannot be captured into a graph",
                     T, vocab);
+    if (!hy::gemm_takes_scratch((int)T, (int)vocab, (int)hidden)) {
+        HIP_TRY(hy::launch_gemm_nt_f32(x, w, resid, out, (int)T, (int)vocab, (int)hidden, s, nullptr));
+        return HY_OK;
+    }
     static std::mutex mu;
     static std::vector<LmScratch> per_dev;
     std::lock_guard<std::mutex> lock(mu);

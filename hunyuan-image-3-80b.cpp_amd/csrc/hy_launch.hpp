@@ -200,7 +200,6 @@ size_t flash_attn_ws_floats(int hd, int slots);
 constexpr int GEMM_SK_GROUPS = 512;     // work groups of the small-batch product: two per CU
 constexpr int GEMM_SPLIT_GROUPS = 256;  // of the larger one: one per CU
 size_t gemm_nt_f32_ws_bytes(int max_rows);
-bool gemm_nt_f32_uses_ws(int M, int N, int K);
 hipError_t launch_gemm_nt_f32(const float* A, const float* W, const float* R, float* C, int M, int N, int K,
                               hipStream_t s, float* ws = nullptr);
 // the same product for 17..128 rows of A (hy_gemm.hip), K a multiple of 32; without ws one

@@ -76,4 +76,14 @@ inline bool norm_in_registers(int T, int H) {
     return H % 256 == 0 && H <= 256 * RMSW_MAX_CHUNKS && (H > 1024 || T <= 2048);
 }
 
+// The stand-alone fp32 product (hy_lm_head_f32): sizes of 64 to 1023 tiles of 128 x 128, which
+// cut tiles between work groups and are refused under stream capture; and those of them that
+// use the shared scratch -- not the decode-sized ones, a stream over W without pieces.
+constexpr int GEMM_GEMV_ROWS = 16;
+inline bool gemm_mid_size(int M, int N, int K) {
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    return K % 32 == 0 && tiles >= 64 && tiles < 1024 && tiles * (K / 32) >= 2048;
+}
+inline bool gemm_takes_scratch(int M, int N, int K) { return M > GEMM_GEMV_ROWS && gemm_mid_size(M, N, K); }
+
 }  // namespace hy

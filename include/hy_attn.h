@@ -150,10 +150,11 @@ int hy_model_forward_hidden(hy_model_ctx* ctx, const float* inputs_embeds_dev, u
  * fp32: fp32 FMAs and MFMAs, or six products of three-way bf16 splits of the operands
  * where these are exact (every value from 2^-110 to 2^127, and smaller ones whose bits
  * end at 2^-133; other values are multiplied by fp32 MFMAs).  x [T][hidden], w
- * [vocab][hidden], all device memory; hidden a multiple of 16.  Mid-size shapes split the reduction over a per-device scratch that the
- * library allocates on first use and orders between calls with an event: those shapes
- * return HY_ERR_UNSUPPORTED under stream capture (hy_model_forward, whose context
- * owns its scratch, can be captured). */
+ * [vocab][hidden], all device memory; hidden a multiple of 16.  Mid-size shapes (64 to 1023 tiles of 128 x 128) of more
+ * than 16 rows split the reduction over a per-device scratch (134 MB) that the library
+ * allocates on first use and orders between calls with an event.  Under stream capture
+ * every shape of that size, whatever its rows, returns HY_ERR_UNSUPPORTED
+ * (hy_model_forward, whose context owns its scratch, can be captured). */
 int hy_lm_head_f32(const float* x_dev, const float* w_dev, const float* resid_dev, uint32_t T, uint32_t hidden,
                    uint32_t vocab, float* out_dev, void* stream);
 

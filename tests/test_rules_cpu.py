@@ -15,6 +15,8 @@ extern "C" int gemv_batch(int wt, unsigned T, int K, int E, int H, int I, int sh
 extern "C" int few_batch(int wt, int T, int K, int E, int I, int sh, int cached) {
     return hy::few_batch(wt, T, K, E, I, sh, cached != 0);
 }
+extern "C" int gemm_mid_size(int M, int N, int K) { return hy::gemm_mid_size(M, N, K); }
+extern "C" int gemm_takes_scratch(int M, int N, int K) { return hy::gemm_takes_scratch(M, N, K); }
 extern "C" int norm_in_registers(int T, int H) { return hy::norm_in_registers(T, H); }
 """
 Q4, Q8 = 2, 8
@@ -123,3 +125,15 @@ def test_norm_kernel(rules, H, T, regs, wave):
 
 def test_norm_registers_hold_the_row(rules):
     assert not any(rules.norm_in_registers(5, H) for H in (64, 1088, 4100, 4352, 8192))
+
+
+def test_decode_lm_head_takes_no_scratch(rules):
+    """One to 16 rows stream over W; more rows of a mid-size grid are cut into pieces."""
+    for N, K in ((32000, 2048), (128256, 4096), (8192, 1024)):
+        assert rules.gemm_mid_size(1, N, K) and not rules.gemm_takes_scratch(1, N, K)
+        assert rules.gemm_mid_size(16, N, K) and not rules.gemm_takes_scratch(16, N, K)
+        assert not rules.gemm_mid_size(17, N, K) or rules.gemm_takes_scratch(17, N, K)
+    for M, N, K in ((256, 4096, 1024), (1290, 6150, 1024), (17, 32000, 2048)):
+        assert rules.gemm_mid_size(M, N, K) and rules.gemm_takes_scratch(M, N, K)
+    for M, N, K in ((256, 4095, 1040), (100, 512, 4096), (4096, 65536, 4096), (128, 8192, 32)):
+        assert not rules.gemm_mid_size(M, N, K) and not rules.gemm_takes_scratch(M, N, K)
