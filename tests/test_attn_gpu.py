@@ -272,11 +272,12 @@ def test_gemm_both_tilings(gpu, M, N, Kd):
     and without the residual, against float64:
       * decode-sized GEMV, M <= 16 (one or two passes over W, ragged N, K not a multiple
         of the 256-float chunk a wave loads);
-      * one-wave register kernel: small grids (17x100, 300x512, 1111x6144 with K=64);
-      * LDS-staged, one 128 x 128 tile per work group: >= 1024 tiles (2100x8200), or
-        K % 32 != 0 with >= 512 tiles (1300x6200x80, stages of 16 floats);
-      * LDS-staged stream-K + fix-up: 64..1023 tiles with K % 32 == 0 (2048x4096x512,
-        1290x6150x4096, 520x6150x1024)."""
+      * one-wave register kernel: grids too small to fill the chip with whole tiles and
+        without scratch (17x100, 300x512, 1111x6144 with K=64);
+      * the bf16-piece kernel, whole tiles: >= 1024 tiles of 128 x 128 (2100x8200), or
+        K % 32 != 0 (1300x6200x80);
+      * the same with tiles cut between work groups: 64..1023 tiles with K % 32 == 0
+        (2048x4096x512, 1290x6150x4096, 520x6150x1024)."""
     rng = np.random.default_rng(M)
     x = rng.standard_normal((M, Kd)).astype(np.float32)
     w = rng.standard_normal((N, Kd)).astype(np.float32)
