@@ -50,7 +50,10 @@ def test_decode_full_shape(gpu, full_layers, ctxs, wt, T):
     assert_exact(out, ref, f"decode wt={wt} T={T}")
 
 
-@pytest.mark.parametrize("wt,T", [(O.Q8_0, 512), (O.Q4_0, 4096), (O.Q8_0, 100)])
+# 48 to 208 tokens: the stream over weights larger than the Infinity Cache (26 pairs per
+# expert end at T = 208), for both types
+@pytest.mark.parametrize("wt,T", [(O.Q8_0, 512), (O.Q4_0, 4096), (O.Q8_0, 100), (O.Q4_0, 48), (O.Q4_0, 208),
+                                  (O.Q4_0, 209), (O.Q8_0, 208), (O.Q8_0, 209)])
 def test_prefill_full_shape_sampled(gpu, full_layers, ctxs, wt, T):
     x = O.synth(200 + T, 0, O.T_X, 0, (T, H), 1.0)
     out, lg, w, idx = ctxs[wt].run(0, x, debug=True)

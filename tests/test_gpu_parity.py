@@ -261,7 +261,8 @@ def test_layer_small(gpu, small_layers, wtype, T):
     m.close()
 
 
-# with E=16, K=4 the grouped GEMM tiles 64 pairs up to T=383 and 128 pairs from T=384
+# with E=16, K=4 and weights this small the grouped GEMM takes 32-pair tiles up to T=256, 64-pair
+# tiles up to T=383 and 128-pair tiles from T=384
 DECODE = dict(H=768, I=768, E=64, K=8)
 
 
@@ -330,13 +331,14 @@ def test_decode_gemv_ring(gpu, wtype, H, I, shared):
 
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_0])
 def test_mfma_narrow_hidden(gpu, wtype):
-    """H = 128 fits only the 128-row tile shape: small batches must still run on it."""
+    """H = 128 fits no 256-row tile: past the stream's 64 pairs per expert (T = 256), and below
+    the 96 (T = 384) from which every width takes the 128-row shape, batches run on that."""
     H, I, E, K = 128, 128, 8, 2
     layer = O.synth_layer(H, I, E, K, wtype, seed=21, std=0.05)
-    m = gpu.Moe(H, I, E, K, wtype, max_tokens=256)
+    m = gpu.Moe(H, I, E, K, wtype, max_tokens=384)
     m.set_path(gpu.PATH_MFMA)
     m.upload(0, layer)
-    for T in (5, 40, 256):
+    for T in (5, 40, 256, 257, 383, 384):
         x = O.synth(70 + T, 0, O.T_X, 0, (T, H), 1.0)
         assert_exact(m.run(0, x), O.moe_forward_q(layer, x), f"H=128 wtype={wtype} T={T}")
     m.close()
