@@ -16,6 +16,18 @@
 
 namespace hy {
 
+// Both products cut their tiles x stages units into p.G contiguous ranges of p.qd units, the
+// first p.rem of one more: first unit of range g, and the range that unit u falls in.
+template <class P>
+__device__ __forceinline__ int gs_lo(const P& p, int g) {
+    return g * p.qd + min(g, p.rem);
+}
+template <class P>
+__device__ __forceinline__ int gs_owner(const P& p, int u) {
+    const int big = p.rem * (p.qd + 1);
+    return u < big ? u / (p.qd + 1) : p.rem + (u - big) / p.qd;
+}
+
 // ---------------------------------------------------------------- small batches (M <= 128)
 // A stream over W: a work group of four waves takes all M rows of A (MT tiles of 32) times
 // 128 rows of W, 32 per wave.  A wave loads its W rows straight into registers in MFMA
@@ -49,13 +61,6 @@ struct GemmSmallArgs {
     int qd, rem;     // tiles x stages = G qd + rem: the first rem ranges take qd + 1 units
     float* part;     // 2 G slots of MT x 32 x 128 floats (unused when G = tiles)
 };
-
-// first unit of range g, and the range unit u falls in
-__device__ __forceinline__ int gs_lo(const GemmSmallArgs& p, int g) { return g * p.qd + min(g, p.rem); }
-__device__ __forceinline__ int gs_owner(const GemmSmallArgs& p, int u) {
-    const int big = p.rem * (p.qd + 1);
-    return u < big ? u / (p.qd + 1) : p.rem + (u - big) / p.qd;
-}
 
 // LDS of one A stage: three pieces of 4 k-chunks of 8 (chunk 2 u + h holds floats
 // 16 u + 4 h .. + 3 and 16 u + 8 + 4 h .. + 3 of a row, the k-slots of MFMA lane half h
@@ -333,11 +338,6 @@ struct GemmSplitArgs {
     int qd, rem;     // tiles x stages = G qd + rem: the first rem ranges take qd + 1 units
     float* part;     // 2 G slots of MT x 64 x 256 floats (unused when G = tiles)
 };
-__device__ __forceinline__ int gs_lo(const GemmSplitArgs& p, int g) { return g * p.qd + min(g, p.rem); }
-__device__ __forceinline__ int gs_owner(const GemmSplitArgs& p, int u) {
-    const int big = p.rem * (p.qd + 1);
-    return u < big ? u / (p.qd + 1) : p.rem + (u - big) / p.qd;
-}
 // row and column tile of tile t
 __device__ __forceinline__ void gs_tile(const GemmSplitArgs& p, int t, int& m, int& n) {
     const int sg = t / (8 * p.nt), r = t - sg * 8 * p.nt, mw = min(8, p.mt - 8 * sg);
@@ -633,8 +633,7 @@ hipError_t launch_gemm_split(const float* A, const float* W, const float* R, flo
     // with scratch: one work group per CU, eight stages each at least
     const int G = !ws ? tiles : U < 8 * GEMM_SPLIT_GROUPS ? (U + 7) / 8 : GEMM_SPLIT_GROUPS;
     const GemmSplitArgs p{A, W, R, C, M, N, K, 32 * sub, mt, nt, G, U / G, U % G, ws};
-    switch ((sub + 1) / 2) {
-    case 1:
+    switch ((sub + 1) / 2) {  // more than 64 rows: three subtiles at least
     case 2: return gemm_split_launch<2>(p, s);
     case 3: return gemm_split_launch<3>(p, s);
     default: return gemm_split_launch<4>(p, s);
