@@ -38,7 +38,7 @@ __device__ __forceinline__ v16f_t mfma_f32(float a, float b, v16f_t c) {
 
 // ---------------------------------------------------------------- GEMM (NT)
 // WM x WN waves per work group, each a 64 x 64 output tile (launched as 1 x 1: the
-// grids too small for the LDS-staged kernel below)
+// grids that hy_gemm.hip does not take)
 template <int WM, int WN>
 __global__ __launch_bounds__(WAVE * WM * WN) void gemm_nt_f32_kernel(const float* __restrict__ A,
                                                                     const float* __restrict__ W,
@@ -391,7 +391,7 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a) {
 // wave covers the whole group for a block of keys, and the keys spread over as many
 // waves as the chip holds.  Every wave is a work group of its own and takes cb
 // consecutive key blocks of one group: K and V of a block reach its own LDS buffer by
-// DMA, in the prompt kernel's swizzled layout, read by the same MFMA steps.  The wave
+// DMA, swizzled as below, and its MFMA steps read them from there.  The wave
 // writes unnormalised O, running max and sum of its 4T live rows;
 // flash_decode_merge_kernel joins the waves of a group.
 // K / V blocks of 32 keys reach LDS by DMA.  Rows are HD floats (HD / 4 16-byte chunks),

@@ -660,6 +660,7 @@ bool mfma_path_ok(int wtype, int H, int I) {
 // weight byte over 128 pairs wins.
 int mfma_shape(int wtype, int T, int K, int E, int H, int I, int has_shared) {
     const int64_t pairs = (int64_t)T * K;
+    // of E + 1 matrices; a launch asks the same of the quants of the matrices it has
     const bool cached = (size_t)(E + 1) * 2 * I * (H / QK) * block_bytes(wtype) <= INFINITY_CACHE;
     if (few_batch(wtype, T, K, E, I, has_shared, cached)) return MM_SHAPE_FEW;
     const bool tall = shape_fits<ShapeTall>(H, I) && pairs < (int64_t)96 * E;

@@ -22,10 +22,10 @@
 #include "hy_lds.hpp"
 
 // Bound: HBM (each expert's weights once per tile) while tiles hold up to ~32 pairs, the
-// fp32 matrix cores beyond: 16 experts of top-4 and the shared one, 4096 x 3072 (2.57 GB),
-// T = 32: 509 us for both products (5.0 TB/s), T = 96: 600 us, T = 512: 1.84 ms (105
-// TFLOP/s).  The decode GEMV, which took these batches before, reads the weights once per
-// four pairs: 910 us, 2.1 ms, 10.7 ms.
+// fp32 matrix cores beyond.  Whole layers of 16 experts of top-4 and the shared one,
+// 4096 x 3072 (2.57 GB; T = 96 fetches 2.66 GB): T = 32 522 us, T = 96 558 us (both products
+// 537 at best, 5.0 TB/s), T = 512 1.85 ms (105 TFLOP/s).  The decode GEMV, which took these
+// batches before, reads the weights once per four pairs: 910 us, 2.06 ms, 10.6 ms.
 namespace hy {
 
 constexpr int MF_RING = 3;  // stages of one block: two in flight while one is consumed
@@ -161,13 +161,16 @@ __global__ __launch_bounds__(256, 2) void moe_mfma_f32_kernel(MfArgs a) {
     }
 }
 
-// 32-pair tiles while experts see up to 32 pairs each: 16 experts of top-4, T = 96: 638
-// against 674 us with 64-pair tiles, 32: 542 against 544; T = 512: 1987 against 1881
+// 32-pair tiles while experts see up to 32 pairs each.  Layers of 16 experts of top-4, 32- against
+// 64-pair tiles: T = 96 558 / 600 us, 128 716 / 707, 160 899 / 780, 512 1981 / 1845.
 int mfma_f32_tokens(int T, int K, int E) { return (int64_t)T * K <= 32 * (int64_t)E ? 32 : 64; }
 
-// The decode GEMV (4 pairs per pass over an expert's weights) stays the better one up to
-// about 3 pairs per expert: 64 experts of top-8, T = 16: 1.43 against 1.48 ms; 16 experts
-// of top-4, T = 8: 458 against 536 us, T = 16: 604 against 539 us, T = 96: 2125 against 638.
+// The decode GEMV (4 pairs per pass over an expert's weights) stays the better one up to about
+// 3 pairs per expert.  Layers of 4096 x 3072, GEMV against these products: 64 experts of top-8
+// T = 16 1.43 / 1.48 ms; 16 of top-4 T = 16 554 / 514 us, T = 32 910 / 522, T = 96 2062 / 558.
+// Past 32 tokens the shared expert alone takes the GEMV nine passes, and these win however few
+// pairs the routed ones see: 2048 x 1536, 64 experts of top-1 T = 33 210 / 207 us, 48 231 / 221,
+// 16 of top-1 T = 33 193 / 142 (a tie again at T = 64 of 64: 274 / 281).
 bool mfma_f32_ok(int T, int K, int E, int H, int I) {
     if (T <= 32 && (int64_t)T * K <= 3 * (int64_t)E) return false;
     // the activation rows are addressed with 32-bit byte offsets

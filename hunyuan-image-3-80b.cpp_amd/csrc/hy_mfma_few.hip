@@ -10,7 +10,8 @@
 //
 // Bound: HBM (each expert's weights once), with the rescale's 64 vector operations per block
 // and wave close behind.  H 4096, I 3072, E 64, K 8, T = 48: Q4_0 337 us a layer (1.38 GB of
-// weights; the LDS-staged 64-pair tiles 455), Q8_0 471 (2.6 GB; 536).  One tile's results
+// weights, 1.43 GB through the memory fabric by the counters; the LDS-staged 64-pair tiles
+// 455), Q8_0 471 (2.6 GB; 536).  One tile's results
 // at a time keep three waves on a SIMD: three of them four blocks deep run Q4_0 in 354 us
 // where two eight deep take 371.  Non-temporal weight loads take Q8_0 from 525 to 471 and
 // Q4_0 from 354 to 337; where a launch's weights fit the Infinity Cache they stay cached

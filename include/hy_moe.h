@@ -189,9 +189,10 @@ int hy_moe_forward_debug(hy_moe_ctx* ctx, uint32_t layer, const float* x_dev, ui
 int hy_moe_stack_forward(hy_moe_ctx* ctx, uint32_t first_layer, uint32_t n_layers,
                          const float* x_dev, uint32_t T, float eps, float* out_dev, void* stream);
 
-/* Expert-product kernels the forward uses: AUTO (default) takes the int8-MFMA grouped
- * GEMM for T > 16 and the dequant-GEMV (VALU dot4) for decode batches, and for F32
- * weights fp32-MFMA products past ~3 pairs per expert; VALU / MFMA
+/* Expert-product kernels the forward uses: AUTO (default) takes the dequant-GEMV (VALU
+ * dot4) for T <= 16 and beyond that up to ~3 (Q4_0) or ~2 (Q8_0) pairs per expert, 5 or
+ * 2.5 in small layers, and int8-MFMA products for larger batches; F32 weights take
+ * fp32-MFMA products past ~3 pairs per expert or 32 tokens.  VALU / MFMA
  * force one (MFMA needs Q8_0/Q4_0 weights and H, I multiples of 128).  Both compute
  * the same float operations in the same order, so they agree bit for bit.  No
  * counterpart in the reference (which has one scalar path); kept so both paths stay
