@@ -55,7 +55,7 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
 }
 // lost gathers the last remainders' bits; lost_bits(lost) once a split was not exact (a bf16
 // value has the low half of its fp32 bits clear): one operation for two operands, eleven
-// for their split
+// for their split (77 x 6144 x 4096: 165 -> 167 us; 4096 rows: 1.03 ms with and without)
 __device__ __forceinline__ bool lost_bits(uint32_t lost) { return (lost & 0xffffu) != 0; }
 __device__ __forceinline__ Split2 split2(float a, float b, uint32_t& lost) {
     Split2 s;
